@@ -32,7 +32,7 @@ struct GroupedCall {
   bool blocked = false;           // digit and abs planes in the blocked layout
   bool packed = false;            // every problem's residue planes in the packed layout
   int packed_kp = 0;              // problems with Kp at most this (> 0) use the packed layout
-  int f64_tiles = 0;              // native GEMM launch word (tile count, kF64Tile128 for 128 x 128 tiles)
+  int f64_tiles = 0;              // native GEMM launch word (tile count and shape)
   ReconGrid rgrid{};              // compact reconstruct / dot-product grids
   int dot_form = 0;               // the handle's dot-product form override (kDotForm*)
   long long prep_blocks = 0;      // workgroups of the compact prep grid (per split)

@@ -242,9 +242,13 @@ inline size_t flag_bytes(int m, int n, size_t plane_entries) {
 constexpr int kPrepRows = 32, kPrepCols = 8;
 
 // FP64 MFMA grouped GEMM (native routes).  h_ws receives the schedule image; *launch receives the
-// launch word for f64_launch: the tile count in bits 0-29, kF64Tile128 set for 128 x 128 tiles (0:
-// nothing to launch).  tile_mode 0 chooses the tile edge from the group's shapes, 64 or 128 forces it.
-constexpr int kF64Tile128 = 1 << 30;
+// launch word for f64_launch: the tile count in bits 0-27, the tile shape from bit kF64ShapeBit (0:
+// nothing to launch).  tile_mode 0 chooses the shape from the group's problems, 64 or 128 forces square
+// tiles of that edge.
+enum {   // 64 x 64, 128 x 128, 16 x 128, 32 x 128, 32 x 32 with one accumulator chain per wave
+  kF64Tile64 = 0, kF64Tile128 = 1, kF64Tile16 = 2, kF64Tile32 = 3, kF64TileChain = 4, kF64Shapes = 5
+};
+constexpr int kF64ShapeBit = 28, kF64MaxTiles = (1 << kF64ShapeBit) - 1;
 int f64_build_schedule(const F64Problem* h, int num, void* h_ws, size_t ws_bytes, int* launch, size_t* bytes_used,
                        int tile_mode = 0);
 int f64_launch(const F64Problem* d_probs, const void* d_sched, int launch, hipStream_t s);

@@ -3,22 +3,33 @@
 // K_TOO_LARGE, SMALL_K, TINY, UNPROFITABLE, PRECISION) and the two native paths
 // (src/ggemm.cu:102-184, src/ggemm_graph.cu:88-102).
 //
-// One launch per group: T x T output tiles of all problems in one table (same prefix/entry format
-// as the INT8 GEMM), workgroup b takes tile b.  256 threads = 4 waves (2 x 2), wave tile
-// T/2 x T/2 of 16 x 16 blocks of v_mfma_f64_16x16x4f64; K staged 16 deep through LDS (double
-// buffer, XOR-swizzled rows).  Two tile sizes, one per group:
-//   T = 64: 2 x 2 blocks per wave, 32 KB of LDS, five workgroups per compute unit (4 % faster than
-//           four with padded rows) -- small and ragged groups;
-//   T = 128: 4 x 4 blocks per wave, 64 KB of LDS, two workgroups per compute unit: half the
-//           operand traffic per flop and four times the MFMA work per fragment read -- groups
-//           with enough large tiles to fill the GPU twice.
-// Every output entry takes the same k-ordered chain of MFMAs (zero-padded beyond k) at either
-// size, so both give bit-identical results.  Descriptors live in device memory, so a captured
-// graph replays with new pointers after one small H2D.
+// One launch per group: output tiles of all problems in one table, workgroup b takes tile b.  One tile
+// shape per group (f64_build_schedule):
+//   128 x 128: 4 waves, 4 x 4 blocks of 16 x 16 each, 64 KB of LDS, two workgroups per compute unit:
+//            half the operand traffic per flop of the next and four times the MFMA work per fragment
+//            read -- groups that fill their rounds;
+//   64 x 64: 2 x 2 blocks per wave, 32 KB of LDS, five workgroups per compute unit -- the others;
+//   16 x 128, 32 x 128: groups of problems with at most 16 / 32 rows, which stream B once;
+//   32 x 32: one block per wave (f64_chain_kernel) -- few outputs, where one chain per wave is what
+//            fills the GPU.
+// A wave owns the 16-row and 16-column blocks of its tile in turn with the other waves, so the blocks
+// of a tile that hangs over the problem's edge are dealt evenly and the ones outside are skipped.
+// Every output entry takes the same k-ordered chain of MFMAs (zero-padded beyond k) at every shape, so
+// all give bit-identical results.  Descriptors live in device memory, so a captured graph replays
+// with new pointers after one small H2D.
+//
+// What bounds it: the FP64 matrix cores, 64 cycles per v_mfma_f64_16x16x4 (75 TFLOP/s measured on
+// register operands); thin groups, HBM; 32 x 32 tiles, the chain's latency.  Measured before -> after
+// B's stages came in as whole 128-byte lines, partial tiles loaded without a test per element and
+// skipped their outside blocks, neighbouring tiles shared an XCD's L2 and a workgroup's priority rose
+// with its progress (same GPU): 64 x 1024^3, beta 0.5, 2.29 -> 2.18 ms (63 TFLOP/s), 96 x 679x600x515
+// 1.11 -> 0.78 ms, 1024 thin panels (5 or 14 rows, 128 columns, k about 880) 0.317 -> 0.217 ms
+// (4.5 TB/s); on 32 x 32 tiles 500x500x60000 3.95 -> 0.73 ms, 3 x 209x197x10380 0.69 -> 0.13 ms.
 // BLAS semantics: alpha == 0 or k == 0 never reads A or B; beta == 0 never reads C.
 #include <algorithm>
+#include <cmath>
 #include <cstring>
-#include <vector>
+#include <type_traits>
 
 #include "common.hpp"
 
@@ -26,144 +37,234 @@ namespace ggemm {
 namespace {
 
 typedef double v4d __attribute__((ext_vector_type(4)));
+typedef double v2d __attribute__((ext_vector_type(2)));
 // global address space: the descriptor pointers would otherwise compile to flat loads, which also
 // count in lgkmcnt, so every LDS fragment wait would wait for the next stage's prefetch as well
 #define GLOBAL __attribute__((address_space(1)))
 constexpr int kThreads = 256;
 constexpr int kBK = 16;
 
-// LDS column of element (k, c): 16-column blocks XOR-swizzled by k mod 4, so the four k rows a
-// fragment read touches sit in different banks without padding (bits 4-5 only: c stays in [0, T))
-__device__ __forceinline__ int swc(int k, int c) { return c ^ ((k & 3) << 4); }
+// LDS positions without padding.  A tile, k-major: row c of k row k, 16-row blocks XOR-swizzled by
+// k mod 4, so that the four k rows a fragment read touches fall into different banks (a tile of one or
+// two blocks needs less).  B tile, in 16-deep k groups, column-major inside a group (the 16 k of a
+// column are one 128-byte line, stored by eight lanes two k each): 16-byte pairs XOR-swizzled by the
+// column, so that a fragment read (16 columns, the 32 bytes of 4 k each) covers every bank evenly.
+template <int W>
+__device__ __forceinline__ int swa(int k, int c) {
+  return W >= 64 ? c ^ (k & 3) << 4 : W == 32 ? c ^ (k & 1) << 4 : c;
+}
+template <int W>
+__device__ __forceinline__ int swb(int k, int c) {
+  return (k >> 4) * (W * 16) + c * 16 + ((((k & 15) >> 1) ^ (c & 7)) << 1 | (k & 1));
+}
 
-template <int T>
-__global__ void __launch_bounds__(kThreads, T == 64 ? 5 : 2) f64_grouped_kernel(const F64Problem* __restrict__ probs,
-                                                                              const int* __restrict__ sched) {
-  constexpr int FB = T / 32;            // 16 x 16 blocks per wave and dimension
-  constexpr int KS = kThreads / T;      // A loader: k rows per pass over the tile's rows
-  constexpr int NA = kBK / KS;          // A elements per thread
-  constexpr int NB = kBK / KS;          // B elements per thread (consecutive k of one column)
-  __shared__ double sA[2][kBK][T];
-  __shared__ double sB[2][kBK][T];
-  const int tile = blockIdx.x;
+// Workgroup -> tile: the dispatcher deals consecutive workgroups to the XCDs in turn, so chunks of
+// 32 consecutive tiles (which share operand panels) go to one XCD's L2.  The tiles come longest first,
+// so the chunks' order turns from one round of chunks to the next.
+__device__ __forceinline__ int tile_of(int b, int total) {
+  constexpr int kChunk = 32;
+  const int super = b / (kXcds * kChunk) * (kXcds * kChunk);
+  if (super + kXcds * kChunk > total) return b;
+  const int i = b - super;
+  return super + ((i + b / (kXcds * kChunk)) % kXcds) * kChunk + i / kXcds;
+}
+
+// The problem of a tile and the tile's index in it.
+struct TileRef {
+  int problem, local;
+};
+__device__ __forceinline__ TileRef find_tile(const int* __restrict__ sched, int block) {
+  const int tile = tile_of(block, sched[0]);
   const int ne = sched[1];
   const int* prefix = sched + kSchedHdr;
   const int* entry = prefix + ne + 1;
-  int lo = 0, hi = ne - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (prefix[mid] <= tile) lo = mid; else hi = mid - 1;
+  int lo = 0;
+  if (const int per = sched[2]) {   // equal tile counts
+    lo = tile / per;
+  } else {
+    int hi = ne - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (prefix[mid] <= tile) lo = mid; else hi = mid - 1;
+    }
   }
-  const F64Problem P = probs[entry[lo] >> 2];
-  const int local = tile - prefix[lo];
-  const int tiles_m = (P.m + T - 1) / T;
-  const int row0 = (local % tiles_m) * T, col0 = (local / tiles_m) * T;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave & 1, wn = wave >> 1;
+  return TileRef{entry[lo] >> 2, tile - prefix[lo]};
+}
 
-  v4d acc[FB][FB];
+// Stages of BK k of a BM x BN tile's operands, HBM to LDS through the registers of 256 threads.  Thread
+// t: A elements (ar, ak + KSA q); B elements (bk, bk + 1) of column bc + 32 c and 16-deep k group g,
+// q = c + CP g, eight lanes to a column's 128 bytes of the group (one request per line: a thread per
+// 64-byte run of a column came back to each line four times, and the lines of a compute unit's
+// workgroups do not fit its L1).  Rows and columns past the problem read its last one (their outputs
+// are not stored), so only a stage that crosses k needs a test per element.
+template <int BM, int BN, int BK>
+struct Loader {
+  static constexpr int KSA = kThreads / BM, NA = BK / KSA, NB = BN * BK / (2 * kThreads), CP = BN / 32;
+  struct Regs {
+    double a[NA], b[NB][2];
+  };
+  const GLOBAL double* Ag;
+  const GLOBAL double* Bg[CP];
+  size_t lda;
+  int k, ar, ak, bc, bk;
+  __device__ __forceinline__ void init(const F64Problem& P, int row0, int col0, int t) {
+    ar = t % BM, ak = t / BM;
+    bc = t / 8, bk = (t % 8) * 2;
+    k = P.k;
+    lda = (size_t)P.lda;
+    Ag = (const GLOBAL double*)P.A + min(row0 + ar, P.m - 1);
 #pragma unroll
-  for (int i = 0; i < FB; ++i)
+    for (int c = 0; c < CP; ++c)
+      Bg[c] = (const GLOBAL double*)P.B + (size_t)min(col0 + bc + 32 * c, P.n - 1) * (size_t)P.ldb;
+  }
+  __device__ __forceinline__ void load(Regs& r, int kt) const {
+    const int k0 = kt * BK;
+    if (k0 + BK <= k) {
+      const GLOBAL double* pa = Ag + (size_t)(k0 + ak) * lda;
 #pragma unroll
-    for (int j = 0; j < FB; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
+      for (int q = 0; q < NA; ++q) r.a[q] = pa[(size_t)(KSA * q) * lda];
+#pragma unroll
+      for (int q = 0; q < NB; ++q) {
+        r.b[q][0] = Bg[q % CP][k0 + 16 * (q / CP) + bk];
+        r.b[q][1] = Bg[q % CP][k0 + 16 * (q / CP) + bk + 1];
+      }
+      return;
+    }
+#pragma unroll
+    for (int q = 0; q < NA; ++q) {
+      const int kk = k0 + ak + KSA * q;
+      const double v = Ag[(size_t)min(kk, k - 1) * lda];
+      r.a[q] = kk < k ? v : 0.0;
+    }
+#pragma unroll
+    for (int q = 0; q < 2 * NB; ++q) {
+      const int kk = k0 + 16 * (q / 2 / CP) + bk + (q & 1);
+      const double v = Bg[q / 2 % CP][min(kk, k - 1)];
+      r.b[q / 2][q & 1] = kk < k ? v : 0.0;
+    }
+  }
+  __device__ __forceinline__ void store(const Regs& r, double (&sA)[BK][BM], double (&sB)[BK * BN]) const {
+#pragma unroll
+    for (int q = 0; q < NA; ++q) sA[ak + KSA * q][swa<BM>(ak + KSA * q, ar)] = r.a[q];
+#pragma unroll
+    for (int q = 0; q < NB; ++q)
+      *reinterpret_cast<v2d*>(&sB[swb<BN>(16 * (q / CP) + bk, bc + 32 * (q % CP))]) = v2d{r.b[q][0], r.b[q][1]};
+  }
+};
+
+// BM x BN tile, WM waves along the rows and 4 / WM along the columns, OCC workgroups per compute unit
+template <int BM, int BN, int WM, int OCC>
+__global__ void __launch_bounds__(kThreads, OCC) f64_grouped_kernel(const F64Problem* __restrict__ probs,
+                                                                 const int* __restrict__ sched) {
+  constexpr int WN = 4 / WM;
+  constexpr int FM = BM / (16 * WM), FN = BN / (16 * WN);   // 16 x 16 blocks per wave
+  constexpr int BK = kBK;
+  __shared__ double sA[2][BK][BM];
+  __shared__ __align__(16) double sB[2][BK * BN];
+  const TileRef t = find_tile(sched, blockIdx.x);
+  const F64Problem P = probs[t.problem];
+  const int local = t.local;
+  const int tiles_m = (P.m + BM - 1) / BM;
+  const int row0 = (local % tiles_m) * BM, col0 = (local / tiles_m) * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave % WM, wn = wave / WM;
+  // this wave's blocks inside the problem: block i covers rows row0 + 16 (WM i + wm) ..
+  const int nbm = min(FM, max(0, (P.m - row0 - 16 * wm + 16 * WM - 1) / (16 * WM)));
+  const int nbn = min(FN, max(0, (P.n - col0 - 16 * wn + 16 * WN - 1) / (16 * WN)));
+
+  v4d acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
 
   const bool compute = P.alpha != 0.0 && P.k > 0;
   if (compute) {
-    // loaders: A element (ar, ak + KS q), B element (bk + q, bc)
-    const int ar = tid % T, ak = tid / T;
-    const int bc = tid / KS, bk = (tid % KS) * NB;
-    const size_t lda = (size_t)P.lda, ldb = (size_t)P.ldb;
-    const bool arow = row0 + ar < P.m, bcol = col0 + bc < P.n;
-    const GLOBAL double* Ag = (const GLOBAL double*)P.A;
-    const GLOBAL double* Bg = (const GLOBAL double*)P.B;
-    double ra[NA], rb[NB];
-    // full tiles (every row and column inside, k a multiple of the stage) load without bounds
-    // tests from two per-stage base pointers; the values are the same either way
-    const bool full = row0 + T <= P.m && col0 + T <= P.n && P.k % kBK == 0;
-    auto gload = [&](int k0) {
-      if (full) {
-        const GLOBAL double* pa = Ag + (size_t)(row0 + ar) + (size_t)(k0 + ak) * lda;
-        const GLOBAL double* pb = Bg + (size_t)(col0 + bc) * ldb + (size_t)(k0 + bk);
-#pragma unroll
-        for (int q = 0; q < NA; ++q) ra[q] = pa[(size_t)(KS * q) * lda];
-#pragma unroll
-        for (int q = 0; q < NB; ++q) rb[q] = pb[q];
-        return;
-      }
-#pragma unroll
-      for (int q = 0; q < NA; ++q) {
-        const int k = k0 + ak + KS * q;
-        ra[q] = (arow && k < P.k) ? Ag[(size_t)(row0 + ar) + (size_t)k * lda] : 0.0;
-      }
-#pragma unroll
-      for (int q = 0; q < NB; ++q) {
-        const int kb = k0 + bk + q;
-        rb[q] = (bcol && kb < P.k) ? Bg[(size_t)kb + (size_t)(col0 + bc) * ldb] : 0.0;
-      }
-    };
-    auto sstore = [&](int st) {
-#pragma unroll
-      for (int q = 0; q < NA; ++q) sA[st][ak + KS * q][swc(ak + KS * q, ar)] = ra[q];
-#pragma unroll
-      for (int q = 0; q < NB; ++q) sB[st][bk + q][swc(bk + q, bc)] = rb[q];
-    };
-    const int nk = (P.k + kBK - 1) / kBK;
-    gload(0);
-    sstore(0);
-    __syncthreads();
+    Loader<BM, BN, BK> ld;
+    ld.init(P, row0, col0, tid);
+    const int nk = (P.k + BK - 1) / BK;
     const int fr = lane & 15, fk = lane >> 4;
-    for (int kt = 0; kt < nk; ++kt) {
-      if (kt + 1 < nk) gload((kt + 1) * kBK);
-      const int st = kt & 1;
+    // The product is taken transposed (B's columns as the MFMA rows), so that a lane's four results
+    // are four columns of one row and 16 lanes store 16 consecutive rows of a column: 128-byte
+    // segments of C.
+    auto loop = [&](auto edge) {
+      constexpr bool kEdge = decltype(edge)::value;
+      // step s of the stage in buffer st: k = 4 s .. 4 s + 3
+      auto step = [&](int st, int s) {
+        double a[FM], b[FN];
 #pragma unroll
-      for (int s = 0; s < kBK / 4; ++s) {
-        double a[FB], b[FB];
+        for (int i = 0; i < FM; ++i) a[i] = sA[st][4 * s + fk][swa<BM>(fk, (WM * i + wm) * 16 + fr)];
 #pragma unroll
-        for (int i = 0; i < FB; ++i) a[i] = sA[st][4 * s + fk][swc(fk, wm * (T / 2) + i * 16 + fr)];
+        for (int j = 0; j < FN; ++j) b[j] = sB[st][swb<BN>(4 * s + fk, fr) + (WN * j + wn) * 256];
 #pragma unroll
-        for (int j = 0; j < FB; ++j) b[j] = sB[st][4 * s + fk][swc(fk, wn * (T / 2) + j * 16 + fr)];
+        for (int i = 0; i < FM; ++i) {
+          if (kEdge && i >= nbm) break;
 #pragma unroll
-        for (int i = 0; i < FB; ++i)
-#pragma unroll
-          for (int j = 0; j < FB; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
-      }
-      if (kt + 1 < nk) sstore((kt + 1) & 1);
+          for (int j = 0; j < FN; ++j) {
+            if (kEdge && j >= nbn) break;
+            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j], a[i], acc[i][j], 0, 0, 0);
+          }
+        }
+      };
+      typename Loader<BM, BN, BK>::Regs r;
+      ld.load(r, 0);
+      ld.store(r, sA[0], sB[0]);
       __syncthreads();
-    }
+      const int quarter = nk >> 2;
+      for (int kt = 0; kt < nk; ++kt) {
+        // a workgroup's priority rises with its progress: the ones sharing a compute unit drift apart,
+        // and one's epilogue and prologue run under the others' MFMAs
+        if (kt == quarter) __builtin_amdgcn_s_setprio(1);
+        if (kt == 2 * quarter) __builtin_amdgcn_s_setprio(2);
+        if (kt == 3 * quarter) __builtin_amdgcn_s_setprio(3);
+        const int st = kt & 1;
+        if (kt + 1 < nk) ld.load(r, kt + 1);
+#pragma unroll
+        for (int s = 0; s < BK / 4; ++s) step(st, s);
+        if (kt + 1 < nk) ld.store(r, sA[st ^ 1], sB[st ^ 1]);
+        __syncthreads();
+      }
+    };
+    if (nbm == FM && nbn == FN)
+      loop(std::false_type{});
+    else
+      loop(std::true_type{});
   }
-  // D block layout of v_mfma_f64_16x16x4f64: lane l, register r -> row 4 r + l / 16, column l % 16
-  // (four single-row groups; the INT8 / F32 16 x 16 instructions use four consecutive rows instead).
+
+  // D block layout of v_mfma_f64_16x16x4f64: lane l, register r -> MFMA row 4 r + l / 16, column
+  // l % 16 (four single-row groups; the INT8 / F32 16 x 16 instructions use four consecutive rows
+  // instead); transposed, so lane l, register r holds C row l % 16, column 4 r + l / 16 of the block.
   // With beta != 0 the C0 values of a batch of blocks are all loaded before the batch's stores:
   // entry by entry, each C0 load waited for its data before the store (the stores might alias
   // the next loads), one memory round trip per entry.
   const size_t ldc = (size_t)P.ldc;
   GLOBAL double* const Cg = (GLOBAL double*)P.C;
   const bool rd = P.beta != 0.0;
-  constexpr int NBLK = FB * FB, BATCH = NBLK < 8 ? NBLK : 8;
+  constexpr int NBLK = FM * FN, BATCH = NBLK < 8 ? NBLK : 8;
 #pragma unroll
   for (int b0 = 0; b0 < NBLK; b0 += BATCH) {
     double c0[BATCH][4];
 #pragma unroll
     for (int q = 0; q < BATCH; ++q) {
-      const int i = (b0 + q) / FB, j = (b0 + q) % FB;
-      const int col = col0 + wn * (T / 2) + j * 16 + (lane & 15);
-      const int rbase = row0 + wm * (T / 2) + i * 16 + (lane >> 4);
+      const int i = (b0 + q) / FN, j = (b0 + q) % FN;
+      const int row = row0 + (WM * i + wm) * 16 + (lane & 15);
+      const int cbase = col0 + (WN * j + wn) * 16 + (lane >> 4);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = rbase + 4 * r;
-        c0[q][r] = (rd && col < P.n && row < P.m) ? Cg[(size_t)row + (size_t)col * ldc] : 0.0;
+        const int col = cbase + 4 * r;
+        c0[q][r] = (rd && row < P.m && col < P.n) ? Cg[(size_t)row + (size_t)col * ldc] : 0.0;
       }
     }
 #pragma unroll
     for (int q = 0; q < BATCH; ++q) {
-      const int i = (b0 + q) / FB, j = (b0 + q) % FB;
-      const int col = col0 + wn * (T / 2) + j * 16 + (lane & 15);
-      const int rbase = row0 + wm * (T / 2) + i * 16 + (lane >> 4);
-      if (col >= P.n) continue;
+      const int i = (b0 + q) / FN, j = (b0 + q) % FN;
+      const int row = row0 + (WM * i + wm) * 16 + (lane & 15);
+      const int cbase = col0 + (WN * j + wn) * 16 + (lane >> 4);
+      if (row >= P.m) continue;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = rbase + 4 * r;
-        if (row >= P.m) continue;
+        const int col = cbase + 4 * r;
+        if (col >= P.n) continue;
         const double ab = compute ? P.alpha * acc[i][j][r] : 0.0;
         Cg[(size_t)row + (size_t)col * ldc] = !rd ? ab : (compute ? ab + P.beta * c0[q][r] : P.beta * c0[q][r]);
       }
@@ -171,28 +272,100 @@ __global__ void __launch_bounds__(kThreads, T == 64 ? 5 : 2) f64_grouped_kernel(
   }
 }
 
-}  // namespace
+// Few outputs (32 x 32 tiles, 512 threads, one workgroup per compute unit): waves 0-3 run one
+// accumulator chain each -- 16 x 16 outputs, the whole k -- and waves 4-7, one beside each on its SIMD,
+// stream the operands in 128-deep stages, two stages ahead in registers.  A chain takes an MFMA every
+// 64-odd cycles whatever else happens, so the time is k / 4 of them as long as the compute waves issue
+// nothing but fragment reads and MFMAs.
+constexpr int kChainTile = 32, kChainBK = 128;
+__global__ void __launch_bounds__(2 * kThreads, 2) f64_chain_kernel(const F64Problem* __restrict__ probs,
+                                                                  const int* __restrict__ sched) {
+  constexpr int T = kChainTile, BK = kChainBK;
+  __shared__ double sA[2][BK][T];
+  __shared__ __align__(16) double sB[2][BK * T];
+  const TileRef t = find_tile(sched, blockIdx.x);
+  const F64Problem P = probs[t.problem];
+  const int tiles_m = (P.m + T - 1) / T;
+  const int row0 = (t.local % tiles_m) * T, col0 = (t.local / tiles_m) * T;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool compute = P.alpha != 0.0 && P.k > 0;
+  const int nk = compute ? (P.k + BK - 1) / BK : 0;
+  if (wave >= 4) {
+    if (!compute) return;
+    Loader<T, T, BK> ld;
+    ld.init(P, row0, col0, tid - kThreads);
+    typename Loader<T, T, BK>::Regs r0, r1;
+    ld.load(r0, 0);
+    if (nk > 1) ld.load(r1, 1);
+    ld.store(r0, sA[0], sB[0]);
+    __syncthreads();
+    for (int kt = 0; kt < nk; kt += 2) {   // stage kt + 1 to LDS while stage kt is multiplied
+      if (kt + 2 < nk) ld.load(r0, kt + 2);
+      if (kt + 1 < nk) ld.store(r1, sA[1], sB[1]);
+      __syncthreads();
+      if (kt + 1 >= nk) break;
+      if (kt + 3 < nk) ld.load(r1, kt + 3);
+      if (kt + 2 < nk) ld.store(r0, sA[0], sB[0]);
+      __syncthreads();
+    }
+    return;
+  }
+  const int wm = wave & 1, wn = wave >> 1;
+  const int row = row0 + 16 * wm + (lane & 15), cbase = col0 + 16 * wn + (lane >> 4);
+  v4d acc = v4d{0.0, 0.0, 0.0, 0.0};
+  if (compute) {
+    const int fr = lane & 15, fk = lane >> 4;
+    auto step = [&](int st, int s) {
+      const double a = sA[st][4 * s + fk][swa<T>(fk, 16 * wm + fr)];
+      const double b = sB[st][swb<T>(4 * s + fk, fr) + 256 * wn];
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(b, a, acc, 0, 0, 0);   // transposed, as above
+    };
+    __builtin_amdgcn_s_setprio(3);
+    __syncthreads();
+    for (int kt = 0; kt < nk; ++kt) {
+      const int steps = (P.k - kt * BK + 3) / 4;   // the steps past k would add zeros
+      if (steps >= BK / 4) {
+#pragma unroll
+        for (int s = 0; s < BK / 4; ++s) step(kt & 1, s);
+      } else {
+#pragma unroll 4
+        for (int s = 0; s < steps; ++s) step(kt & 1, s);
+      }
+      __syncthreads();
+    }
+  }
+  const size_t ldc = (size_t)P.ldc;
+  GLOBAL double* const Cg = (GLOBAL double*)P.C;
+  const bool rd = P.beta != 0.0;
+  double c0[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    c0[r] = (rd && row < P.m && cbase + 4 * r < P.n) ? Cg[(size_t)row + (size_t)(cbase + 4 * r) * ldc] : 0.0;
+  if (row >= P.m) return;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    if (cbase + 4 * r >= P.n) continue;
+    const double ab = compute ? P.alpha * acc[r] : 0.0;
+    Cg[(size_t)row + (size_t)(cbase + 4 * r) * ldc] = !rd ? ab : (compute ? ab + P.beta * c0[r] : P.beta * c0[r]);
+  }
+}
 
-namespace {
-long long tiles_of(const F64Problem& p, int t) { return (long long)((p.m + t - 1) / t) * ((p.n + t - 1) / t); }
+constexpr int kCus = 256;
+struct F64Shape {
+  int bm, bn;
+};
+constexpr F64Shape kShapes[kF64Shapes] = {{64, 64}, {128, 128}, {16, 128}, {32, 128}, {32, 32}};
+
+long long tiles_of(const F64Problem& p, const F64Shape& t) {
+  return (long long)((p.m + t.bm - 1) / t.bm) * ((p.n + t.bn - 1) / t.bn);
+}
+
 }  // namespace
 
 int f64_build_schedule(const F64Problem* h, int num, void* h_ws, size_t ws_bytes, int* launch, size_t* bytes_used,
                        int tile_mode) {
   if (num < 0 || (num > 0 && !h) || !h_ws || !launch) return 1;
   if (ws_bytes < sched_bytes(num)) return 2;
-  // tile edge: 128 when the 128 x 128 tiles fill two workgroups on each of 256 compute units at
-  // least twice and pad the outputs by at most 1/8 more than 64 x 64 tiles do, else 64
-  int tile = tile_mode == 64 || tile_mode == 128 ? tile_mode : 64;
-  if (tile_mode == 0) {
-    long long t128 = 0, a64 = 0;
-    for (int i = 0; i < num; ++i)
-      if (h[i].m > 0 && h[i].n > 0) {
-        t128 += tiles_of(h[i], 128);
-        a64 += tiles_of(h[i], 64);
-      }
-    if (t128 >= 1024 && 4 * t128 * 8 <= a64 * 9) tile = 128;
-  }
   // problems with outputs, longest k first (ties by index: the order a stable sort keeps), sorted
   // in place in the image's entry array -- no host scratch
   int* img = static_cast<int*>(h_ws);
@@ -200,36 +373,80 @@ int f64_build_schedule(const F64Problem* h, int num, void* h_ws, size_t ws_bytes
   for (int i = 0; i < num; ++i) ne += h[i].m > 0 && h[i].n > 0;
   int* prefix = img + kSchedHdr;
   int* entry = prefix + ne + 1;
-  for (int i = 0, j = 0; i < num; ++i)
-    if (h[i].m > 0 && h[i].n > 0) entry[j++] = i;
+  int mmax = 0, kmax = 0;
+  long long tiles[kF64Shapes] = {};
+  double work128 = 0, area = 0;
+  for (int i = 0, j = 0; i < num; ++i) {
+    const F64Problem& p = h[i];
+    if (p.m <= 0 || p.n <= 0) continue;
+    entry[j++] = i;
+    mmax = std::max(mmax, p.m);
+    const int k = p.alpha == 0.0 ? 0 : p.k;
+    kmax = std::max(kmax, k);
+    for (int s = 0; s < kF64Shapes; ++s) tiles[s] += tiles_of(p, kShapes[s]);
+    work128 += (double)tiles_of(p, kShapes[kF64Tile128]) * k;
+    area += (double)p.m * p.n;
+  }
   std::sort(entry, entry + ne, [h](int a, int b) {
     const int ka = std::max(h[a].k, 1), kb = std::max(h[b].k, 1);
     return ka != kb ? ka > kb : a < b;
   });
+
+  // Tile shape.  Microseconds per 16 k, measured on groups of 1 to 3000 tiles: a round of 32 x 32 tiles
+  // (one per compute unit) 0.22, of 64 x 64 tiles 0.58 but at least 0.85 in all, of the thin ones 1.0 but
+  // at least 1.2 (their problems differ in k, and then a round of 32 x 32 ones takes 0.4).  128 x 128
+  // (67 TFLOP/s on long k against 61 of the 64 x 64 tiles) when little of the tiles hangs over the
+  // problems' edges and their rounds of two workgroups per compute unit are nearly filled: a short last
+  // round leaves compute units idle for as long as a full one, unless it has at most one tile for each.
+  int shape = tile_mode == 128 ? kF64Tile128 : kF64Tile64;
+  if (tile_mode == 0 && kmax > 0) {
+    auto rounds = [&](int s) { return std::ceil((double)tiles[s] / kCus); };
+    if (mmax <= 32) {
+      const int thin = mmax <= 16 ? kF64Tile16 : kF64Tile32;
+      shape = 0.4 * rounds(kF64TileChain) < std::max(1.2, 1.0 * rounds(thin)) ? kF64TileChain : thin;
+    } else if (0.22 * rounds(kF64TileChain) < std::max(0.85, 0.58 * rounds(kF64Tile64))) {
+      shape = kF64TileChain;
+    } else if (area >= 0.95 * 16384.0 * tiles[kF64Tile128]) {
+      const double share = work128 / kmax / (2.0 * kCus);
+      const double full = std::floor(share), left = share - full;
+      if (share >= 0.87 * (full + (left <= 0.0 ? 0.0 : left <= 0.5 ? 0.5 : 1.0))) shape = kF64Tile128;
+    }
+  }
+  const F64Shape& t = kShapes[shape];
   long long tot = 0;
+  bool equal = true;
   for (size_t j = 0; j < ne; ++j) {
-    const F64Problem& p = h[entry[j]];
+    const long long n = tiles_of(h[entry[j]], t);
     prefix[j] = (int)tot;
-    tot += tiles_of(p, tile);
-    entry[j] <<= 2;
+    tot += n;
+    if (tot > kF64MaxTiles) return 5;
+    equal = equal && n == tiles_of(h[entry[0]], t);
   }
   prefix[ne] = (int)tot;
-  if (tot >= kF64Tile128) return 5;
   std::memset(img, 0, sizeof(int) * kSchedHdr);
   img[0] = (int)tot;
   img[1] = (int)ne;
-  *launch = tot == 0 ? 0 : (int)tot | (tile == 128 ? kF64Tile128 : 0);
+  img[2] = ne && equal ? prefix[1] : 0;
+  for (size_t j = 0; j < ne; ++j) entry[j] <<= 2;
+  *launch = tot == 0 ? 0 : (int)tot | shape << kF64ShapeBit;
   if (bytes_used) *bytes_used = sizeof(int) * (kSchedHdr + 2 * ne + 1);
   return 0;
 }
 
 int f64_launch(const F64Problem* d_probs, const void* d_sched, int launch, hipStream_t s) {
   if (launch <= 0) return 0;
-  const unsigned tiles = (unsigned)(launch & (kF64Tile128 - 1));
-  if (launch & kF64Tile128)
-    hipLaunchKernelGGL(f64_grouped_kernel<128>, dim3(tiles), dim3(kThreads), 0, s, d_probs, static_cast<const int*>(d_sched));
-  else
-    hipLaunchKernelGGL(f64_grouped_kernel<64>, dim3(tiles), dim3(kThreads), 0, s, d_probs, static_cast<const int*>(d_sched));
+  const unsigned tiles = (unsigned)(launch & kF64MaxTiles);
+  const int shape = launch >> kF64ShapeBit;
+  const int* sched = static_cast<const int*>(d_sched);
+  if (shape == kF64TileChain) {
+    hipLaunchKernelGGL(f64_chain_kernel, dim3(tiles), dim3(2 * kThreads), 0, s, d_probs, sched);
+  } else {
+    const auto kernel = shape == kF64Tile128  ? f64_grouped_kernel<128, 128, 2, 2>
+                        : shape == kF64Tile16 ? f64_grouped_kernel<16, 128, 1, 4>
+                        : shape == kF64Tile32 ? f64_grouped_kernel<32, 128, 2, 4>
+                                              : f64_grouped_kernel<64, 64, 2, 5>;
+    hipLaunchKernelGGL(kernel, dim3(tiles), dim3(kThreads), 0, s, d_probs, sched);
+  }
   return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 

@@ -1,0 +1,47 @@
+"""The native FP64 GEMM's tile shapes on the edges of tiles, of the 16- and 128-deep k stages and of the
+rule that chooses: 32 x 32 tiles (few outputs), 16 x 128 and 32 x 128 tiles (many thin problems),
+128 x 128 tiles (filled rounds).  Every shape takes the same k-ordered chain per entry, so each result
+equals the 64 x 64 kernel's (forced with GGEMM_F64_TILE) bit for bit; that kernel is held to the
+componentwise gamma_n bound against the host's extended-precision dots."""
+import pytest
+
+import ggemm as G
+from gpu_util import same_bits, say
+from test_gpu_grouped import Case, kernel_handle, run
+
+pytestmark = pytest.mark.gpu
+
+CFG = G.Config(0, 1e-15, 1, G.REPAIR_ON)
+GROUPS = {
+    # few outputs: 32 x 32 tiles
+    "chain_edges": [(32, 32, 128), (33, 31, 127), (31, 33, 129), (64, 1, 255), (1, 64, 256), (70, 50, 257), (1, 1, 1),
+                    (40, 40, 0), (0, 5, 5), (48, 48, 385)],
+    "chain_long_k": [(70, 50, 9000), (65, 1, 8191), (5, 40, 12345)],
+    "chain_alpha0": [(50, 40, 300, 0.0, 0.5), (50, 40, 300, -1.0, 0.0)],
+    # enough thin problems for the thin tiles
+    "thin16": [(1 + i % 16, 120 + i % 20, 1 + i % 50) for i in range(300)],
+    "thin32": [(1 + i % 32, 250 + i % 9, 15 + i % 35) for i in range(300)],
+    # one full round of 128 x 128 tiles per compute unit and no edges
+    "tile128": [(2048, 2048, 40)],
+}
+
+
+@pytest.mark.parametrize("beta", [0.0, -0.5])
+@pytest.mark.parametrize("name", sorted(GROUPS))
+def test_native_shapes(name, beta):
+    say(f"native shapes: {name}, beta {beta}")
+    outs = []
+    for env in ({}, {"GGEMM_F64_TILE": "64"}):
+        case = Case(GROUPS[name], 41, phi=1.0, alpha=1.5, beta=beta)
+        with kernel_handle(case, None, **env) as hd:
+            rc, st = run(case, G.PATH_NATIVE_GROUPED, CFG, handle=hd)
+        assert rc == 0 and st.kernel_launches == 1
+        outs.append([case.C(g).copy() for g in range(len(case.hp))])
+    for g, (a, b) in enumerate(zip(*outs)):
+        assert same_bits(a, b), (g, GROUPS[name][g])
+    for g, h in enumerate(case.hp):
+        if h.m == 0 or h.n == 0 or h.m * h.n * h.k > 10 ** 8:
+            continue
+        h.reference()
+        gate, _ = h.gate(outs[0][g])
+        assert gate <= 1.0, (g, gate)
