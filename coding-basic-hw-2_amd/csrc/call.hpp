@@ -36,6 +36,7 @@ struct GroupedCall {
   ReconGrid rgrid{};              // compact reconstruct / dot-product grids
   int dot_form = 0;               // the handle's dot-product form override (kDotForm*)
   long long prep_blocks = 0;      // workgroups of the compact prep grid (per split)
+  long long prep_elems = 0;       // elements (Kp per row / column) they read
   size_t h2d_bytes = 0;           // bytes of the blob to copy
 };
 

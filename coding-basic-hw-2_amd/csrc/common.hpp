@@ -265,9 +265,11 @@ int f64_launch(const F64Problem* d_probs, const void* d_sched, int launch, hipSt
 // pofs (with order, or nullptr): a compact grid of total_blocks workgroups, problem order[i] owning
 // blocks pofs[i] .. pofs[i + 1] - 1 (ceil(m / 32) A-row blocks, then ceil(n / 8) B-column blocks;
 // none for problems prep skips)
+// elems (with launches): the operands' elements in all; groups of few rows and columns over a long k take
+// two launches, *launches receives the number
 int prep_launch(const oz2_problem* d, int num, int max_m, int max_n, hipStream_t s, int fold_q, int packed_kp,
                 int max_moduli, const YDesc* yd = nullptr, const int* order = nullptr, const int* pofs = nullptr,
-                long long total_blocks = 0);
+                long long total_blocks = 0, long long elems = 0, int* launches = nullptr);
 // yd == nullptr: read the int32 planes of oz2_problem::C32 (kernel-level API); else the digits.
 // blocked: the digits and L of every problem are in the blocked layout (production, yd != nullptr);
 // the reconstruct then flags the entries that take FP64 dot products and a second kernel computes

@@ -436,8 +436,9 @@ int build_grouped(ggemm_handle_t h, const ggemm_problem_t* probs, int num, const
       const oz2_problem& o = pd[po[i]];
       if (tot > 0x7fffffffLL) return GGEMM_ERR_INVALID;
       pof[i] = (int)tot;
-      if (o.alpha != 0.0 && o.num_moduli >= 1 && o.num_moduli <= kMaxModuli)
-        tot += (long long)(o.m + kPrepRows - 1) / kPrepRows + (o.n + kPrepCols - 1) / kPrepCols;
+      if (o.alpha == 0.0 || o.num_moduli < 1 || o.num_moduli > kMaxModuli) continue;
+      c.prep_elems += vol(po[i]);
+      tot += (long long)(o.m + kPrepRows - 1) / kPrepRows + (o.n + kPrepCols - 1) / kPrepCols;
     }
     if (tot > 0x7fffffffLL) return GGEMM_ERR_INVALID;
     c.prep_blocks = tot;
@@ -459,12 +460,14 @@ int enqueue_grouped(const GroupedCall& c, const char* db, hipStream_t s, int rep
   prof::mark(prof_set, 0, s);
   if (c.ne > 0) {
     const bool shared = c.nprep > 0;   // operand reuse: prep once per unique operand
+    int np = 0;
     if (prep_launch(shared ? reinterpret_cast<const oz2_problem*>(db + c.L.off_prep) : doz, shared ? c.nprep : c.ne,
                     shared ? c.pmax_m : c.max_m, shared ? c.pmax_n : c.max_n, s, 1, c.packed_kp, c.nmax,
                     shared ? nullptr : dyd, reinterpret_cast<const int*>(db + c.L.off_po),
-                    reinterpret_cast<const int*>(db + c.L.off_po) + (shared ? c.nprep : c.ne), c.prep_blocks))
+                    reinterpret_cast<const int*>(db + c.L.off_po) + (shared ? c.nprep : c.ne), c.prep_blocks,
+                    c.prep_elems, &np))
       return GGEMM_ERR_NUMERICS;
-    ++*launches;
+    *launches += np;
     prof::mark(prof_set, 1, s);
     if (i8_launch(reinterpret_cast<const i8_problem*>(db + c.L.off_i8), reinterpret_cast<const I8Epi*>(db + c.L.off_epi),
                   db + c.L.off_si8, &c.i8info, s, c.i8_kernel, c.i8_hw))

@@ -235,7 +235,8 @@ __device__ __forceinline__ void nf_header(GLOBAL int32_t* nfw, int ni, int nan, 
 }
 
 // ------------------------------------------------------------------------------- A rows
-template <bool kWide>
+// kNormed: the shifts are there already (norm_kernel), and only this split's residues are written.
+template <bool kWide, bool kNormed>
 __device__ void prep_rows(const oz2_problem& pr, const CrtTables* __restrict__ tab, int blk, int split,
                           int nsplit, PrepShared& sm, unsigned long long* cnt, int widx, bool packed, int32_t* nfo,
                           int* nff, bool zero_nf, const YDesc* yds, int pi) {
@@ -243,7 +244,7 @@ __device__ void prep_rows(const oz2_problem& pr, const CrtTables* __restrict__ t
   // split 0, when the call asks for summaries: pass 1, which reads every value of the block's rows,
   // also collects each row's non-finite summary state (NaN seen, largest finite magnitude,
   // infinity positions); it is written for the rows whose shift turns out non-finite
-  const bool trk = nfo && split == 0;   // block-uniform
+  const bool trk = !kNormed && nfo && split == 0;   // block-uniform
   if (trk) {
     if (tid < kARows) {
       sm.nfcnt[tid] = 0;
@@ -261,102 +262,111 @@ __device__ void prep_rows(const oz2_problem& pr, const CrtTables* __restrict__ t
   const size_t lda = (size_t)pr.lda;
   const double T = tab->T[N];
 
-  // ---- pass 1: row max and sum of squares, chain c = k mod 8 ascending.  With trk, mx is the
-  // largest FINITE magnitude and every infinity is listed instead; the row max is then infinite
-  // exactly when the row's infinity count is nonzero, so the shift is the same
-  double mx = 0.0, ss = 0.0;
-  auto step = [&](double a, int k) {
-    ss = fma(a, a, ss);
-    if (!trk) {
-      mx = fmax(mx, fabs(a));
-      return;
+  if constexpr (kNormed) {
+    if (c == 0) {
+      sm.shift[r] = valid ? ((const GLOBAL int32_t*)pr.row_shift)[i] : 0;
+      sm.sig[r] = valid ? ((const GLOBAL int32_t*)pr.row_shift)[m + i] : OZ2_SHIFT_ZERO;
     }
-    const double aa = fabs(a);
-    const bool inf = aa == __builtin_inf();
-    mx = fmax(mx, inf ? 0.0 : aa);
-    if (inf) {   // rare: the summary's address is formed here, not kept live through the pass
-      const int x = atomicAdd(&sm.nfcnt[r], 1);
-      if (x < kNfCap) ((GLOBAL int32_t*)nfo)[(size_t)kNfWords * i + 2 + x] = k | (a < 0.0 ? (int)0x80000000u : 0);
-    }
-  };
-  if (valid) {
-    int k = c;
-    // groups of 16 k per chain, software-pipelined: the next group's loads are issued before this
-    // group's chain, so 16 to 32 loads stay in flight (a long-k block is one of few workgroups and
-    // streams megabytes); the load past the last group re-reads it (in bounds) so that the load
-    // count between two waits is the same on every path
-    auto ld16 = [&](double (&a)[16], int k0) {
-#pragma unroll
-      for (int t = 0; t < 16; ++t) a[t] = A[i + (size_t)(k0 + 8 * t) * lda];
-    };
-    auto chain16 = [&](const double (&a)[16], int k0) {
-#pragma unroll
-      for (int t = 0; t < 16; ++t) step(a[t], k0 + 8 * t);
-    };
-    if (k + 8 * 15 < K) {
-      double a[16], b[16];
-      ld16(a, k);
-      for (;;) {
-        bool more = k + 8 * 31 < K;
-        ld16(b, more ? k + 128 : k);
-        chain16(a, k);
-        k += 128;
-        if (!more) break;
-        more = k + 8 * 31 < K;
-        ld16(a, more ? k + 128 : k);
-        chain16(b, k);
-        k += 128;
-        if (!more) break;
-      }
-    }
-    for (; k < K; k += 8) step(A[i + (size_t)k * lda], k);
-    if (trk && isnan(ss)) sm.nfnan[r] = 1;   // a sum of squares turns NaN only through a NaN
-  }
-  sm.red0[c][r] = mx;
-  __syncthreads();
-  if (c == 0) {
-    double M = 0.0;
-    for (int q = 0; q < kChains; ++q) M = fmax(M, sm.red0[q][r]);
-    if (trk) {   // M is the largest finite magnitude: the summary's, and infinite row max if any Inf
-      sm.nfmx[r] = (unsigned long long)__double_as_longlong(M);
-      if (sm.nfcnt[r] > 0) M = __builtin_inf();
-    }
-    sm.rowmax[r] = M;
-  }
-  __syncthreads();
-  const double rowmax = sm.rowmax[r];
-  // (an infinite row max already makes the shift non-finite: no rescaled second read of the row)
-  const bool resc = valid && isfinite(rowmax) && needs_rescale(rowmax);
-  if (resc) {   // rare: exact power-of-two prescaling so the squares cannot overflow / underflow
-    const int e = -ilogb(rowmax);
-    ss = 0.0;
-    for (int k = c; k < K; k += kChains) {
-      const double a = mul_pow2(A[i + (size_t)k * lda], e);
+    __syncthreads();
+  } else {
+    // ---- pass 1: row max and sum of squares, chain c = k mod 8 ascending.  With trk, mx is the
+    // largest FINITE magnitude and every infinity is listed instead; the row max is then infinite
+    // exactly when the row's infinity count is nonzero, so the shift is the same
+    double mx = 0.0, ss = 0.0;
+    auto step = [&](double a, int k) {
       ss = fma(a, a, ss);
+      if (!trk) {
+        mx = fmax(mx, fabs(a));
+        return;
+      }
+      const double aa = fabs(a);
+      const bool inf = aa == __builtin_inf();
+      mx = fmax(mx, inf ? 0.0 : aa);
+      if (inf) {   // rare: the summary's address is formed here, not kept live through the pass
+        const int x = atomicAdd(&sm.nfcnt[r], 1);
+        if (x < kNfCap) ((GLOBAL int32_t*)nfo)[(size_t)kNfWords * i + 2 + x] = k | (a < 0.0 ? (int)0x80000000u : 0);
+      }
+    };
+    if (valid) {
+      int k = c;
+      // groups of 16 k per chain, software-pipelined: the next group's loads are issued before this
+      // group's chain, so 16 to 32 loads stay in flight (a long-k block is one of few workgroups and
+      // streams megabytes); the load past the last group re-reads it (in bounds) so that the load
+      // count between two waits is the same on every path
+      auto ld16 = [&](double (&a)[16], int k0) {
+  #pragma unroll
+        for (int t = 0; t < 16; ++t) a[t] = A[i + (size_t)(k0 + 8 * t) * lda];
+      };
+      auto chain16 = [&](const double (&a)[16], int k0) {
+  #pragma unroll
+        for (int t = 0; t < 16; ++t) step(a[t], k0 + 8 * t);
+      };
+      if (k + 8 * 15 < K) {
+        double a[16], b[16];
+        ld16(a, k);
+        for (;;) {
+          bool more = k + 8 * 31 < K;
+          ld16(b, more ? k + 128 : k);
+          chain16(a, k);
+          k += 128;
+          if (!more) break;
+          more = k + 8 * 31 < K;
+          ld16(a, more ? k + 128 : k);
+          chain16(b, k);
+          k += 128;
+          if (!more) break;
+        }
+      }
+      for (; k < K; k += 8) step(A[i + (size_t)k * lda], k);
+      if (trk && isnan(ss)) sm.nfnan[r] = 1;   // a sum of squares turns NaN only through a NaN
     }
-  }
-  sm.red1[c][r] = ss;
-  __syncthreads();
-  if (c == 0) {
-    double S = 0.0;
-    for (int q = 0; q < kChains; ++q) S += sm.red1[q][r];
-    const int sh = valid ? shift_from_norm(rowmax, S, resc, T) : 0;
-    const int sg = valid ? abs_shift(rowmax, sh) : OZ2_SHIFT_ZERO;
-    sm.shift[r] = sh;
-    sm.sig[r] = sg;
-    if (valid && split == 0) {
-      ((GLOBAL int32_t*)pr.row_shift)[i] = sh;
-      ((GLOBAL int32_t*)pr.row_shift)[m + i] = sg;
-      if (sh == OZ2_SHIFT_NONFINITE) {
-        atomicAdd(counter_slot(cnt), 1ull);
-        if (nff) *nff = 1;   // (every writer stores the same value)
+    sm.red0[c][r] = mx;
+    __syncthreads();
+    if (c == 0) {
+      double M = 0.0;
+      for (int q = 0; q < kChains; ++q) M = fmax(M, sm.red0[q][r]);
+      if (trk) {   // M is the largest finite magnitude: the summary's, and infinite row max if any Inf
+        sm.nfmx[r] = (unsigned long long)__double_as_longlong(M);
+        if (sm.nfcnt[r] > 0) M = __builtin_inf();
+      }
+      sm.rowmax[r] = M;
+    }
+    __syncthreads();
+    const double rowmax = sm.rowmax[r];
+    // (an infinite row max already makes the shift non-finite: no rescaled second read of the row)
+    const bool resc = valid && isfinite(rowmax) && needs_rescale(rowmax);
+    if (resc) {   // rare: exact power-of-two prescaling so the squares cannot overflow / underflow
+      const int e = -ilogb(rowmax);
+      ss = 0.0;
+      for (int k = c; k < K; k += kChains) {
+        const double a = mul_pow2(A[i + (size_t)k * lda], e);
+        ss = fma(a, a, ss);
       }
     }
+    sm.red1[c][r] = ss;
+    __syncthreads();
+    if (c == 0) {
+      double S = 0.0;
+      for (int q = 0; q < kChains; ++q) S += sm.red1[q][r];
+      const int sh = valid ? shift_from_norm(rowmax, S, resc, T) : 0;
+      const int sg = valid ? abs_shift(rowmax, sh) : OZ2_SHIFT_ZERO;
+      sm.shift[r] = sh;
+      sm.sig[r] = sg;
+      if (valid && split == 0) {
+        ((GLOBAL int32_t*)pr.row_shift)[i] = sh;
+        ((GLOBAL int32_t*)pr.row_shift)[m + i] = sg;
+        if (sh == OZ2_SHIFT_NONFINITE) {
+          atomicAdd(counter_slot(cnt), 1ull);
+          if (nff) *nff = 1;   // (every writer stores the same value)
+        }
+      }
+    }
+    __syncthreads();
+    // the rows' finite flags (the descriptor is formed here, not kept live through the pass)
+    uint8_t* const frw = (split == 0 && yds) ? yds[pi].fr : nullptr;
+    if (frw && tid < kARows && row0 + tid < m) frw[row0 + tid] = sm.shift[tid] != OZ2_SHIFT_NONFINITE ? 1 : 0;
+
   }
-  __syncthreads();
-  // the rows' finite flags (the descriptor is formed here, not kept live through the pass)
-  uint8_t* const frw = (split == 0 && yds) ? yds[pi].fr : nullptr;
-  if (frw && tid < kARows && row0 + tid < m) frw[row0 + tid] = sm.shift[tid] != OZ2_SHIFT_NONFINITE ? 1 : 0;
 
   // ---- pass 2: residues of this split's k-tiles; split 0 also walks every tile for the
   //      ordered ||dA||, ||A'|| chain sums (the residue values do not depend on the split)
@@ -371,7 +381,8 @@ __device__ void prep_rows(const oz2_problem& pr, const CrtTables* __restrict__ t
   const int ntile = (Kp + kATile - 1) / kATile;
   const int per = (ntile + nsplit - 1) / nsplit;
   const int w0 = min(ntile, split * per), w1 = min(ntile, w0 + per);   // tiles written here
-  int l0 = split == 0 ? 0 : w0, l1 = split == 0 ? ntile : w1;   // tiles walked here
+  const bool sums = !kNormed && split == 0;
+  int l0 = sums ? 0 : w0, l1 = sums ? ntile : w1;   // tiles walked here
   // without zero residues, a block whose every row is non-finite has nothing to walk (its rows'
   // sums stay 0, as the walk leaves them)
   if (!zero_nf && __syncthreads_and(!valid || nf_c)) l1 = l0;
@@ -383,7 +394,7 @@ __device__ void prep_rows(const oz2_problem& pr, const CrtTables* __restrict__ t
       const int k = k0 + c + kChains * jj;
       av[jj] = (valid && !nf_c && k < K) ? A[i + (size_t)k * lda] : 0.0;
     }
-    if (!nf_c && split == 0) {
+    if (!nf_c && sums) {
       double xs[kATile / kChains];
       scaled<kATile / kChains>(av, sh_c, xs);
 #pragma unroll
@@ -424,7 +435,7 @@ __device__ void prep_rows(const oz2_problem& pr, const CrtTables* __restrict__ t
     }
     __syncthreads();
   }
-  if (split != 0) return;   // block-uniform
+  if (!sums) return;   // block-uniform
   sm.red0[c][r] = da2;
   sm.red1[c][r] = na2;
   __syncthreads();
@@ -440,7 +451,7 @@ __device__ void prep_rows(const oz2_problem& pr, const CrtTables* __restrict__ t
 // ---------------------------------------------------------------------------- B columns
 constexpr int kBReg = 32;   // column values per lane held in registers (K <= 32 kBReg: one read of B)
 
-template <bool kWide>
+template <bool kWide, bool kNormed>
 __device__ void prep_cols(const oz2_problem& pr, const CrtTables* __restrict__ tab, int blk, int split,
                           int nsplit, PrepShared& sm, unsigned long long* cnt, bool packed, int32_t* nfo, int* nff,
                           bool zero_nf, const YDesc* yds, int pi) {
@@ -448,6 +459,30 @@ __device__ void prep_cols(const oz2_problem& pr, const CrtTables* __restrict__ t
   const int j = blk * kBCols + w;
   const int n = pr.n, N = pr.num_moduli, K = pr.k, Kp = pr.kp;
   if (j >= n) return;   // no barriers below; the 32-lane group is column-uniform
+  if constexpr (kNormed) {   // this split's residues only
+    const GLOBAL double* __restrict__ b = (const GLOBAL double*)pr.B + (size_t)j * pr.ldb;
+    const int sh = ((const GLOBAL int32_t*)pr.col_shift)[j], sg = ((const GLOBAL int32_t*)pr.col_shift)[n + j];
+    if (sh == OZ2_SHIFT_NONFINITE) return;   // (the grouped pipeline leaves these residues unwritten)
+    const int nchunk = (Kp + 127) / 128, per = (nchunk + nsplit - 1) / nsplit;
+    const int c0 = min(nchunk, split * per), c1 = min(nchunk, c0 + per);
+    for (int ch = c0; ch < c1; ++ch) {
+      const int k0 = 128 * ch + 4 * lane;
+      if (k0 >= Kp) continue;
+      double a[4], xt[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a[e] = (k0 + e < K) ? b[k0 + e] : 0.0;
+      scaled<4>(a, sh, xt);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) xt[e] = trunc(xt[e]);
+      GLOBAL int8_t* const base = (GLOBAL int8_t*)pr.B8 + (packed ? packed_offset(j, k0, n, Kp) : (size_t)j * Kp + k0);
+      planes<4, kWide>(xt, N, tab, 0, base, pr.b8_mod_stride);
+      uint32_t q = 0u;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) q |= abs_u8(a[e], sg) << (8 * e);
+      *(GLOBAL uint32_t*)(base + (size_t)N * pr.b8_mod_stride) = q;
+    }
+    return;
+  }
   if (nfo && lane == 0) {   // the column's summary state (used by this 32-lane group only)
     sm.nfcnt[w] = 0;
     sm.nfnan[w] = 0;
@@ -679,6 +714,264 @@ __device__ void prep_cols(const oz2_problem& pr, const CrtTables* __restrict__ t
   }
 }
 
+// ------------------------------------------------------- long-k groups: norms, then residues
+// Few rows and columns over a long k (prep_two_pass): the ordered chains are the only serial part, so
+// they run by themselves, one wave for 8 rows (lane = row + 8 chain) or 2 columns, with 32 to 64 loads
+// in flight per lane -- first the norms (norm_kernel), then beside the residues, which any number of
+// workgroups may share once the shifts are known, the sums of ||dA|| and ||A'|| (walk_*).  Same
+// chains, same order and so the same bits as prep_rows / prep_cols.
+constexpr int kDeep = 32;
+// f(value, k) over this lane's k = k0, k0 + step, ..., < K of p[k * stride]
+template <class F>
+__device__ __forceinline__ void walk_chain(const GLOBAL double* p, size_t stride, int k0, int step, int K, F f) {
+  int k = k0;
+  auto ld = [&](double (&a)[kDeep], int kk) {
+#pragma unroll
+    for (int t = 0; t < kDeep; ++t) a[t] = p[(size_t)(kk + step * t) * stride];
+  };
+  auto run = [&](const double (&a)[kDeep], int kk) {
+#pragma unroll
+    for (int t = 0; t < kDeep; ++t) f(a[t], kk + step * t);
+  };
+  const int span = step * kDeep, last = step * (kDeep - 1);
+  if (k + last < K) {
+    double a[kDeep], b[kDeep];
+    ld(a, k);
+    for (;;) {   // a load past the last whole group re-reads this one
+      bool more = k + span + last < K;
+      ld(b, more ? k + span : k);
+      run(a, k);
+      k += span;
+      if (!more) break;
+      more = k + span + last < K;
+      ld(a, more ? k + span : k);
+      run(b, k);
+      k += span;
+      if (!more) break;
+    }
+  }
+  for (; k < K; k += step) f(p[(size_t)k * stride], k);
+}
+
+struct NormShared {
+  int cnt[8], nan[8];
+};
+// Shift words, finite flag and non-finite summary of one row (8 lanes, slot = row) or column (32 lanes):
+// mx the lane's largest finite magnitude, ss its chain's sum of squares.
+struct NormOut {
+  int32_t* shift;        // the operand's shift words
+  int n, i;              // its rows / columns, this one
+  const GLOBAL double* p;
+  size_t stride;
+  int32_t* nfw;          // summary, or nullptr
+  uint8_t* finite;       // finite flags, or nullptr
+};
+template <bool kRows>
+__device__ void norm_wave(const NormOut& o, bool valid, int K, double T, NormShared& sm, unsigned long long* cnt, int* nff) {
+  const int lane = threadIdx.x & 63;
+  const int c = kRows ? lane >> 3 : lane & 31, slot = kRows ? lane & 7 : lane >> 5;
+  constexpr int kStep = kRows ? kChains : 32;
+  if (lane < 8) sm.cnt[lane] = sm.nan[lane] = 0;
+  __syncthreads();
+  double mx = 0.0, ss = 0.0;
+  if (valid)
+    walk_chain(o.p, o.stride, c, kStep, K, [&](double a, int k) {
+      ss = fma(a, a, ss);
+      const double aa = fabs(a);
+      const bool inf = aa == __builtin_inf();
+      mx = fmax(mx, inf ? 0.0 : aa);
+      if (inf) {
+        const int x = atomicAdd(&sm.cnt[slot], 1);
+        if (o.nfw && x < kNfCap) ((GLOBAL int32_t*)o.nfw)[2 + x] = k | (a < 0.0 ? (int)0x80000000u : 0);
+      }
+    });
+  if (isnan(ss)) sm.nan[slot] = 1;   // a sum of squares turns NaN only through a NaN
+  __syncthreads();
+  double M = mx;   // the largest finite magnitude
+  if (kRows) {
+    for (int q = 0; q < kChains; ++q) M = fmax(M, __shfl(mx, slot + 8 * q));
+  } else {
+#pragma unroll
+    for (int h = 16; h; h >>= 1) M = fmax(M, __shfl_xor(M, h, 32));
+  }
+  const double rowmax = sm.cnt[slot] > 0 ? __builtin_inf() : M;
+  const bool resc = valid && isfinite(rowmax) && needs_rescale(rowmax);
+  if (resc) {   // rare: exact power-of-two prescaling so the squares cannot overflow / underflow
+    const int e = -ilogb(rowmax);
+    ss = 0.0;
+    for (int k = c; k < K; k += kStep) {
+      const double a = mul_pow2(o.p[(size_t)k * o.stride], e);
+      ss = fma(a, a, ss);
+    }
+  }
+  double S = 0.0;
+  if (kRows) {
+    for (int q = 0; q < kChains; ++q) S += __shfl(ss, slot + 8 * q);
+  } else {
+    S = ss;
+#pragma unroll
+    for (int h = 16; h; h >>= 1) S += __shfl_xor(S, h, 32);
+  }
+  if (!valid || c != 0) return;
+  const int sh = shift_from_norm(rowmax, S, resc, T);
+  GLOBAL int32_t* const w = (GLOBAL int32_t*)o.shift;
+  w[o.i] = sh;
+  w[o.n + o.i] = abs_shift(rowmax, sh);
+  const bool nf = sh == OZ2_SHIFT_NONFINITE;
+  if (nf) {
+    atomicAdd(counter_slot(cnt), 1ull);
+    if (nff) *nff = 1;
+    if (o.nfw)
+      nf_header((GLOBAL int32_t*)o.nfw, sm.cnt[slot], sm.nan[slot], (unsigned long long)__double_as_longlong(M));
+  }
+  if (o.finite) o.finite[o.i] = nf ? 0 : 1;
+}
+
+// ||dA|| and ||A'|| of 8 rows / 2 columns, from the shifts norm_kernel wrote.
+__device__ __forceinline__ void walk_step(double a, int sh, double sc, double& da2, double& na2) {
+  const double x = sh >= -1000 && sh <= 1000 ? a * sc : mul_pow2(a, sh), xt = trunc(x), fr = x - xt;
+  da2 = fma(fr, fr, da2);
+  na2 = fma(xt, xt, na2);
+}
+__device__ void walk_rows(const oz2_problem& pr, int row0) {
+  const int lane = threadIdx.x & 63, slot = lane & 7, c = lane >> 3;
+  const int i = row0 + slot, m = pr.m;
+  GLOBAL int32_t* const w = (GLOBAL int32_t*)pr.row_shift;
+  const int sh = i < m ? w[i] : OZ2_SHIFT_NONFINITE;
+  double da2 = 0.0, na2 = 0.0;
+  if (sh != OZ2_SHIFT_NONFINITE) {
+    const double sc = pow2d(max(-1000, min(1000, sh)));
+    walk_chain((const GLOBAL double*)pr.A + i, (size_t)pr.lda, c, kChains, pr.k,
+               [&](double a, int) { walk_step(a, sh, sc, da2, na2); });
+  }
+  double D = 0.0, Nn = 0.0;
+  for (int q = 0; q < kChains; ++q) {
+    D += __shfl(da2, slot + 8 * q);
+    Nn += __shfl(na2, slot + 8 * q);
+  }
+  if (c == 0 && i < m) {
+    w[2 * m + i] = norm_ub_bits(D);
+    w[3 * m + i] = norm_ub_bits(Nn);
+  }
+}
+__device__ void walk_cols(const oz2_problem& pr, int col0) {
+  const int lane = threadIdx.x & 31, j = col0 + ((threadIdx.x & 63) >> 5), n = pr.n, K = pr.k;
+  if (j >= n) return;
+  GLOBAL int32_t* const w = (GLOBAL int32_t*)pr.col_shift;
+  const int sh = w[j];
+  double da2 = 0.0, na2 = 0.0;
+  if (sh != OZ2_SHIFT_NONFINITE) {
+    const double sc = pow2d(max(-1000, min(1000, sh)));
+    const GLOBAL double* const b = (const GLOBAL double*)pr.B + (size_t)j * pr.ldb;
+    constexpr int kG = 8;   // chunks of 128 k in flight, twice
+    auto ld = [&](double (&a)[4 * kG], int k0) {
+#pragma unroll
+      for (int t = 0; t < 4 * kG; ++t) a[t] = b[k0 + 128 * (t / 4) + 4 * lane + (t & 3)];
+    };
+    auto run = [&](const double (&a)[4 * kG]) {
+#pragma unroll
+      for (int t = 0; t < 4 * kG; ++t) walk_step(a[t], sh, sc, da2, na2);
+    };
+    int k = 0;
+    if (128 * kG <= K) {
+      double a[4 * kG], c[4 * kG];
+      ld(a, 0);
+      for (;;) {
+        bool more = k + 2 * 128 * kG <= K;
+        ld(c, more ? k + 128 * kG : k);
+        run(a);
+        k += 128 * kG;
+        if (!more) break;
+        more = k + 2 * 128 * kG <= K;
+        ld(a, more ? k + 128 * kG : k);
+        run(c);
+        k += 128 * kG;
+        if (!more) break;
+      }
+    }
+    for (; k < K; k += 128)
+      for (int e = 0; e < 4; ++e)
+        if (k + 4 * lane + e < K) walk_step(b[k + 4 * lane + e], sh, sc, da2, na2);
+  }
+#pragma unroll
+  for (int h = 16; h; h >>= 1) {
+    da2 += __shfl_xor(da2, h, 32);
+    na2 += __shfl_xor(na2, h, 32);
+  }
+  if (lane == 0) {
+    w[2 * n + j] = norm_ub_bits(da2);
+    w[3 * n + j] = norm_ub_bits(na2);
+  }
+}
+
+// The block's problem in the compact grid: the last one whose first block is at most blk (empty problems
+// are skipped); blk becomes the block's index in it.
+__device__ __forceinline__ int compact_problem(const int* __restrict__ order, const int* __restrict__ pofs, int nprob,
+                                               int& blk) {
+  int lo = 0, hi = nprob - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (pofs[mid] <= blk) lo = mid; else hi = mid - 1;
+  }
+  blk -= pofs[lo];
+  return order[lo];
+}
+
+// Four one-wave workgroups for each block of the compact grid: 8 of its 32 rows or 2 of its 8 columns.
+__global__ void __launch_bounds__(64, 2) norm_kernel(const oz2_problem* __restrict__ probs,
+                                                  const CrtTables* __restrict__ tab, unsigned long long* __restrict__ cnt,
+                                                  const YDesc* __restrict__ yds, const int* __restrict__ order,
+                                                  const int* __restrict__ pofs, int nprob) {
+  __shared__ NormShared sm;
+  int blk = (int)blockIdx.x >> 2;
+  const int sub = (int)blockIdx.x & 3, pi = compact_problem(order, pofs, nprob, blk);
+  const oz2_problem& pr = probs[pi];
+  const int N = pr.num_moduli;
+  if (N < 1 || N > kMaxModuli || pr.alpha == 0.0) return;
+  const int a_blocks = (pr.m + kARows - 1) / kARows;
+  int32_t* const nfo = yds ? yds[pi].nf : nullptr;
+  int* const nff = yds ? const_cast<int*>(&yds[pi].nff) : nullptr;
+  const int lane = threadIdx.x;
+  if (blk < a_blocks) {
+    const int i = blk * kARows + 8 * sub + (lane & 7);
+    const bool valid = i < pr.m;
+    const NormOut o{pr.row_shift, pr.m, i, (const GLOBAL double*)pr.A + (valid ? i : 0), (size_t)pr.lda,
+                    nfo ? nfo + (size_t)kNfWords * i : nullptr, yds ? yds[pi].fr : nullptr};
+    norm_wave<true>(o, valid, pr.k, tab->T[N], sm, cnt, nff);
+  } else {
+    const int j = (blk - a_blocks) * kBCols + 2 * sub + (lane >> 5);
+    const bool valid = j < pr.n;
+    const NormOut o{pr.col_shift, pr.n, j, (const GLOBAL double*)pr.B + (valid ? (size_t)j * pr.ldb : 0), 1,
+                    nfo ? nfo + (size_t)kNfWords * ((size_t)pr.m + j) : nullptr, yds ? yds[pi].fc : nullptr};
+    norm_wave<false>(o, valid, pr.k, tab->T[N], sm, cnt, nff);
+  }
+}
+
+// blockIdx.y = 0: the sums of one block of the compact grid; else residue split y - 1 of it.
+template <bool kWide>
+__global__ void __launch_bounds__(kThreads, 4) residue_kernel(const oz2_problem* __restrict__ probs,
+                                                           const CrtTables* __restrict__ tab, int packed_kp,
+                                                           const int* __restrict__ order, const int* __restrict__ pofs,
+                                                           int nprob) {
+  __shared__ PrepShared sm;
+  int blk = (int)blockIdx.x;
+  const oz2_problem& pr = probs[compact_problem(order, pofs, nprob, blk)];
+  const int N = pr.num_moduli;
+  if (N < 1 || N > kMaxModuli || pr.alpha == 0.0) return;
+  const int a_blocks = (pr.m + kARows - 1) / kARows;
+  const bool packed = pr.kp <= packed_kp, rows = blk < a_blocks;
+  const int split = (int)blockIdx.y - 1, nsplit = (int)gridDim.y - 1;
+  if (split < 0) {
+    const int wave = threadIdx.x >> 6;
+    if (rows) walk_rows(pr, blk * kARows + 8 * wave);
+    else walk_cols(pr, (blk - a_blocks) * kBCols + 2 * wave);
+  } else if (rows) {
+    prep_rows<kWide, true>(pr, tab, blk, split, nsplit, sm, nullptr, N, packed, nullptr, nullptr, false, nullptr, 0);
+  } else {
+    prep_cols<kWide, true>(pr, tab, blk - a_blocks, split, nsplit, sm, nullptr, packed, nullptr, nullptr, false, nullptr, 0);
+  }
+}
+
 // kWide: three-word digits (any N); the two-word kernel is launched only for calls whose every
 // problem has T_N < 1.5 2^62.
 // Grid: compact (pofs != nullptr) -- blockIdx.x runs over the real blocks of all problems, problem
@@ -694,14 +987,8 @@ __global__ void __launch_bounds__(kThreads, 4) prep_kernel(const oz2_problem* __
                                                         int nprob) {
   __shared__ PrepShared sm;
   int pi, blk = (int)blockIdx.x;
-  if (pofs) {   // the last problem whose first block is at most blockIdx.x (empty problems are skipped)
-    int lo = 0, hi = nprob - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (pofs[mid] <= blk) lo = mid; else hi = mid - 1;
-    }
-    pi = order[lo];
-    blk -= pofs[lo];
+  if (pofs) {
+    pi = compact_problem(order, pofs, nprob, blk);
     a_blocks = (probs[pi].m + kARows - 1) / kARows;
   } else {
     pi = order ? order[blockIdx.y] : (int)blockIdx.y;
@@ -722,18 +1009,25 @@ __global__ void __launch_bounds__(kThreads, 4) prep_kernel(const oz2_problem* __
   const bool zero_nf = !fold_q;
   if (blk < a_blocks) {
     if (blk * kARows >= pr.m) return;
-    prep_rows<kWide>(pr, tab, blk, blockIdx.z, gridDim.z, sm, cnt, fold ? N : 0, packed, nfo, nff, zero_nf, yds, pi);
+    prep_rows<kWide, false>(pr, tab, blk, blockIdx.z, gridDim.z, sm, cnt, fold ? N : 0, packed, nfo, nff, zero_nf, yds, pi);
   } else {
-    prep_cols<kWide>(pr, tab, blk - a_blocks, blockIdx.z, gridDim.z, sm, cnt, packed, nfo, nff, zero_nf, yds, pi);
+    prep_cols<kWide, false>(pr, tab, blk - a_blocks, blockIdx.z, gridDim.z, sm, cnt, packed, nfo, nff, zero_nf, yds, pi);
   }
 }
 
 int g_force_split = 0;
 
+// Whether a grouped call's prep takes two launches (norm_kernel, residue_kernel): at most two of the
+// single kernel's workgroups per compute unit without its k splits, each of which reads its rows'
+// whole k again, and enough elements (16 M, 128 MB) that the second launch does not matter.
+bool prep_two_pass(long long blocks, long long elems, int cus) { return blocks <= 2LL * cus && elems >= 1LL << 24; }
+
 }  // namespace
 
 int prep_launch(const oz2_problem* d, int num, int max_m, int max_n, hipStream_t s, int fold_q, int packed_kp,
-                int max_moduli, const YDesc* yd, const int* order, const int* pofs, long long total_blocks) {
+                int max_moduli, const YDesc* yd, const int* order, const int* pofs, long long total_blocks,
+                long long elems, int* launches) {
+  if (launches) *launches = 0;
   if (num <= 0) return 0;
   if (num > 65535 || max_m < 0 || max_n < 0 || max_moduli < 1 || max_moduli > kMaxModuli) return 1;
   if (pofs && (!order || total_blocks < 0 || total_blocks > 0x7fffffffLL)) return 1;
@@ -751,7 +1045,20 @@ int prep_launch(const oz2_problem* d, int num, int max_m, int max_n, hipStream_t
   const CrtTables* ht = host_tables();
   if (!ht) return 2;
   const dim3 g3(grid.x, grid.y, S);
-  if (ht->T[max_moduli] < 0x1.8p62)
+  const bool wide = !(ht->T[max_moduli] < 0x1.8p62);
+  if (launches) *launches = 1;
+  if (launches && pofs && fold_q && g_force_split == 0 && prep_two_pass(blocks, elems, c->num_cus)) {
+    hipLaunchKernelGGL(norm_kernel, dim3(4 * (unsigned)blocks), dim3(64), 0, s, d, c->tab, c->counters, yd, order, pofs, num);
+    const unsigned Sr = (unsigned)std::min<long long>(64, (8LL * c->num_cus + blocks - 1) / blocks);
+    const dim3 gr((unsigned)blocks, 1 + Sr);
+    if (wide)
+      hipLaunchKernelGGL(residue_kernel<true>, gr, dim3(kThreads), 0, s, d, c->tab, packed_kp, order, pofs, num);
+    else
+      hipLaunchKernelGGL(residue_kernel<false>, gr, dim3(kThreads), 0, s, d, c->tab, packed_kp, order, pofs, num);
+    *launches = 2;
+    return hipGetLastError() == hipSuccess ? 0 : 3;
+  }
+  if (!wide)
     hipLaunchKernelGGL(prep_kernel<false>, g3, dim3(kThreads), 0, s, d, a_blocks, c->tab, c->counters, fold_q,
                        packed_kp, yd, order, pofs, num);
   else
