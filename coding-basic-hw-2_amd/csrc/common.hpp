@@ -26,7 +26,6 @@ struct CrtTables {
   int32_t p[kMaxModuli];
   uint32_t magic[kMaxModuli];                  // floor(2^32 / p)
   float ipf[kMaxModuli];                       // 1 / p, nearest float
-  float cf[kMaxModuli];                        // (floor(p / 2) + 1/2) / p + 2048, nearest float
   // byte weights of the digit words, four per word, for word kind k:
   //   k = 0: unsigned bytes 2^(8 i) mod p, i = 0..3        (low word, unsigned digits)
   //   k = 1: unsigned bytes 2^(8 i) mod p, i = 4..7        (wide middle word, unsigned digits)

@@ -108,7 +108,6 @@ int build(CrtTables* t) {
     t->p[l] = (int32_t)p;
     t->magic[l] = (uint32_t)((1ull << 32) / p);
     t->ipf[l] = (float)(1.0 / (double)p);
-    t->cf[l] = (float)(((double)(p / 2) + 0.5) / (double)p + 2048.0);
     digit_weights(p, 1u, t->wb[0][l]);
   }
   for (int N = 1; N <= kMaxModuli; ++N) {

@@ -106,16 +106,16 @@ __device__ __forceinline__ int32_t norm_ub_bits(double x) {
 // planes):
 //   u = v_dot4_u32_u8 over L (and M), then v_dot4_i32_i8 over H; u = x (mod p) and
 //       -2^16 <= u < 2^19 + 2^16 (unsigned words give [0, 8 255^2], the signed one [-2^16, 2^16])
-//   q = trunc(fmaf(u, ipf, cf)) = floor((u + h) / p) + 2048, h = floor(p / 2), where ipf and
-//       cf = (h + 1/2)/p + 2048 are the nearest floats: the exact value (u + h + 1/2)/p + 2048 is
-//       positive and below 2^13, its fractional part (j + 1/2)/p is at least 1/(2p) >= 2^-9 from an
-//       integer, and the computed one is within |u| 2^-32 + 2^-13 + 2^-12 < 2^-10 of it (checked
-//       exhaustively over every u and p on the host)
-//   r = u - q p = sym(x mod p) - 2048 p, and 2048 p = 0 (mod 256): its low byte is the stored
-//       byte of the symmetric residue in [-h, p - 1 - h]
-// Full-rate 32-bit operations only: two or three dot products, three float operations and one
-// 24-bit multiply-add per residue, no table lookups.  The bytes equal the reference's
-// reduce / negate / symmetric-map sequence (sym(x mod p) is unique).
+//   q = rint(u / p), as the low 24 bits of fmaf(u, ipf, 1.5 2^23), which hold 2^22 + q: ipf is the
+//       nearest float to 1 / p; u / p is at least 1/(2p) >= 2^-9 from a half-integer for odd p and
+//       u ipf within 2^-12 of it, and the fma rounds once, to an integer (checked exhaustively over
+//       every u and p on the host).  For p = 256 any q will do.
+//   r = u - (2^22 + q) p = sym(u mod p) - 2^22 p, and 2^22 p = 0 (mod 256): its low byte is the stored
+//       byte of the symmetric residue in [-floor(p / 2), p - 1 - floor(p / 2)]
+// Full-rate 32-bit operations only: two or three dot products, two float operations and one 24-bit
+// multiply-add per residue, no table lookups (taking q from a truncating conversion was one more; same
+// GPU, 64 x 1024^3 per call 2650 -> 2630 us, 16 x 1536x512x2048 with one A 714 -> 702).  The bytes
+// equal the reference's reduce / negate / symmetric-map sequence (sym(x mod p) is unique).
 template <bool kWide>
 struct Digits {
   uint32_t w[kWide ? 3 : 2];   // L, (M,) balanced H
@@ -136,12 +136,12 @@ __device__ __forceinline__ Digits<kWide> digits_of(double x) {
 struct PlaneW {
   uint32_t w0, w1;
   int wh, p;
-  float ip, c;
+  float ip;
 };
 template <bool kWide>
 __device__ __forceinline__ PlaneW plane_w(const CrtTables* __restrict__ tab, int l, int widx) {
   const uint32_t* w = tab->wb[widx][l];
-  return PlaneW{w[0], w[1], (int)w[kWide ? 3 : 2], tab->p[l], tab->ipf[l], tab->cf[l]};
+  return PlaneW{w[0], w[1], (int)w[kWide ? 3 : 2], tab->p[l], tab->ipf[l]};
 }
 __device__ __forceinline__ uint32_t pack4(int r0, int r1, int r2, int r3) {   // low bytes
   const uint32_t lo = __builtin_amdgcn_perm((uint32_t)r1, (uint32_t)r0, 0x0c0c0400u);
@@ -166,7 +166,7 @@ __device__ __forceinline__ void residue_bytes(const Digits<kWide>* x, const Plan
 #pragma unroll
     for (int e = 0; e < G; ++e) u[e] = __builtin_amdgcn_sdot4((int)x[g + e].w[kWide ? 2 : 1], k.wh, (int)s[e], false);
 #pragma unroll
-    for (int e = 0; e < G; ++e) r[e] = (int)__builtin_fmaf((float)u[e], k.ip, k.c);
+    for (int e = 0; e < G; ++e) r[e] = __float_as_int(__builtin_fmaf((float)u[e], k.ip, 0x1.8p23f));
 #pragma unroll
     for (int e = 0; e < G; ++e) r[e] = __mul24(r[e], -k.p) + u[e];
 #pragma unroll
@@ -716,13 +716,13 @@ __device__ void prep_cols(const oz2_problem& pr, const CrtTables* __restrict__ t
 
 // ------------------------------------------------------- long-k groups: norms, then residues
 // Few rows and columns over a long k (prep_two_pass): the ordered chains are the only serial part, so
-// they run by themselves, one wave for 8 rows (lane = row + 8 chain) or 2 columns, with 32 to 64 loads
-// in flight per lane -- first the norms (norm_kernel), then beside the residues, which any number of
-// workgroups may share once the shifts are known, the sums of ||dA|| and ||A'|| (walk_*).  Same
-// chains, same order and so the same bits as prep_rows / prep_cols.
-constexpr int kDeep = 32;
+// they run by themselves -- first the norms (norm_kernel), then beside the residues, which any number
+// of workgroups may share once the shifts are known, the sums of ||dA|| and ||A'|| (walk_*).  Same
+// chains, same order and so the same bits as prep_rows / prep_cols.  Bound by the requests a compute
+// unit keeps in flight: 16 rows x 4 chains per wave, so that each is a whole 128-byte line of A
+// (8 rows x 8 chains, 64 bytes: 267 against 264 us for 2 x 984 rows and columns of 40000), and kDeep to 2 kDeep loads in flight per lane.
 // f(value, k) over this lane's k = k0, k0 + step, ..., < K of p[k * stride]
-template <class F>
+template <int kDeep, class F>
 __device__ __forceinline__ void walk_chain(const GLOBAL double* p, size_t stride, int k0, int step, int K, F f) {
   int k = k0;
   auto ld = [&](double (&a)[kDeep], int kk) {
@@ -753,11 +753,12 @@ __device__ __forceinline__ void walk_chain(const GLOBAL double* p, size_t stride
   for (; k < K; k += step) f(p[(size_t)k * stride], k);
 }
 
+constexpr int kNormThreads = 128, kNormRows = 16, kNormCols = 4;
 struct NormShared {
-  int cnt[8], nan[8];
+  int cnt[kNormRows], nan[kNormRows];
+  double red0[kChains][kNormRows], red1[kChains][kNormRows];
 };
-// Shift words, finite flag and non-finite summary of one row (8 lanes, slot = row) or column (32 lanes):
-// mx the lane's largest finite magnitude, ss its chain's sum of squares.
+// Shift words, finite flag and non-finite summary of a row (8 lanes) or a column (32 lanes).
 struct NormOut {
   int32_t* shift;        // the operand's shift words
   int n, i;              // its rows / columns, this one
@@ -767,15 +768,15 @@ struct NormOut {
   uint8_t* finite;       // finite flags, or nullptr
 };
 template <bool kRows>
-__device__ void norm_wave(const NormOut& o, bool valid, int K, double T, NormShared& sm, unsigned long long* cnt, int* nff) {
-  const int lane = threadIdx.x & 63;
-  const int c = kRows ? lane >> 3 : lane & 31, slot = kRows ? lane & 7 : lane >> 5;
+__device__ void norm_group(const NormOut& o, bool valid, int K, double T, NormShared& sm, unsigned long long* cnt, int* nff) {
+  const int tid = threadIdx.x;
+  const int c = kRows ? tid >> 4 : tid & 31, slot = kRows ? tid & 15 : tid >> 5;
   constexpr int kStep = kRows ? kChains : 32;
-  if (lane < 8) sm.cnt[lane] = sm.nan[lane] = 0;
+  if (tid < kNormRows) sm.cnt[tid] = sm.nan[tid] = 0;
   __syncthreads();
   double mx = 0.0, ss = 0.0;
   if (valid)
-    walk_chain(o.p, o.stride, c, kStep, K, [&](double a, int k) {
+    walk_chain<32>(o.p, o.stride, c, kStep, K, [&](double a, int k) {
       ss = fma(a, a, ss);
       const double aa = fabs(a);
       const bool inf = aa == __builtin_inf();
@@ -786,10 +787,11 @@ __device__ void norm_wave(const NormOut& o, bool valid, int K, double T, NormSha
       }
     });
   if (isnan(ss)) sm.nan[slot] = 1;   // a sum of squares turns NaN only through a NaN
+  if (kRows) sm.red0[c][slot] = mx;
   __syncthreads();
   double M = mx;   // the largest finite magnitude
   if (kRows) {
-    for (int q = 0; q < kChains; ++q) M = fmax(M, __shfl(mx, slot + 8 * q));
+    for (int q = 0; q < kChains; ++q) M = fmax(M, sm.red0[q][slot]);
   } else {
 #pragma unroll
     for (int h = 16; h; h >>= 1) M = fmax(M, __shfl_xor(M, h, 32));
@@ -806,7 +808,9 @@ __device__ void norm_wave(const NormOut& o, bool valid, int K, double T, NormSha
   }
   double S = 0.0;
   if (kRows) {
-    for (int q = 0; q < kChains; ++q) S += __shfl(ss, slot + 8 * q);
+    sm.red1[c][slot] = ss;
+    __syncthreads();
+    for (int q = 0; q < kChains; ++q) S += sm.red1[q][slot];
   } else {
     S = ss;
 #pragma unroll
@@ -833,29 +837,31 @@ __device__ __forceinline__ void walk_step(double a, int sh, double sc, double& d
   da2 = fma(fr, fr, da2);
   na2 = fma(xt, xt, na2);
 }
-__device__ void walk_rows(const oz2_problem& pr, int row0) {
-  const int lane = threadIdx.x & 63, slot = lane & 7, c = lane >> 3;
+__device__ void walk_rows(const oz2_problem& pr, int row0, PrepShared& sm) {   // 32 rows, 256 threads
+  const int tid = threadIdx.x, c = (tid >> 4) & 7, slot = (tid & 15) + 16 * (tid >> 7);
   const int i = row0 + slot, m = pr.m;
   GLOBAL int32_t* const w = (GLOBAL int32_t*)pr.row_shift;
   const int sh = i < m ? w[i] : OZ2_SHIFT_NONFINITE;
   double da2 = 0.0, na2 = 0.0;
   if (sh != OZ2_SHIFT_NONFINITE) {
     const double sc = pow2d(max(-1000, min(1000, sh)));
-    walk_chain((const GLOBAL double*)pr.A + i, (size_t)pr.lda, c, kChains, pr.k,
-               [&](double a, int) { walk_step(a, sh, sc, da2, na2); });
+    walk_chain<16>((const GLOBAL double*)pr.A + i, (size_t)pr.lda, c, kChains, pr.k,
+                   [&](double a, int) { walk_step(a, sh, sc, da2, na2); });
   }
+  sm.red0[c][slot] = da2;
+  sm.red1[c][slot] = na2;
+  __syncthreads();
+  if (c != 0 || i >= m) return;
   double D = 0.0, Nn = 0.0;
   for (int q = 0; q < kChains; ++q) {
-    D += __shfl(da2, slot + 8 * q);
-    Nn += __shfl(na2, slot + 8 * q);
+    D += sm.red0[q][slot];
+    Nn += sm.red1[q][slot];
   }
-  if (c == 0 && i < m) {
-    w[2 * m + i] = norm_ub_bits(D);
-    w[3 * m + i] = norm_ub_bits(Nn);
-  }
+  w[2 * m + i] = norm_ub_bits(D);
+  w[3 * m + i] = norm_ub_bits(Nn);
 }
-__device__ void walk_cols(const oz2_problem& pr, int col0) {
-  const int lane = threadIdx.x & 31, j = col0 + ((threadIdx.x & 63) >> 5), n = pr.n, K = pr.k;
+__device__ void walk_cols(const oz2_problem& pr, int col0) {   // 8 columns, 256 threads
+  const int lane = threadIdx.x & 31, j = col0 + (threadIdx.x >> 5), n = pr.n, K = pr.k;
   if (j >= n) return;
   GLOBAL int32_t* const w = (GLOBAL int32_t*)pr.col_shift;
   const int sh = w[j];
@@ -863,7 +869,7 @@ __device__ void walk_cols(const oz2_problem& pr, int col0) {
   if (sh != OZ2_SHIFT_NONFINITE) {
     const double sc = pow2d(max(-1000, min(1000, sh)));
     const GLOBAL double* const b = (const GLOBAL double*)pr.B + (size_t)j * pr.ldb;
-    constexpr int kG = 8;   // chunks of 128 k in flight, twice
+    constexpr int kG = 4;   // chunks of 128 k in flight, twice
     auto ld = [&](double (&a)[4 * kG], int k0) {
 #pragma unroll
       for (int t = 0; t < 4 * kG; ++t) a[t] = b[k0 + 128 * (t / 4) + 4 * lane + (t & 3)];
@@ -917,33 +923,33 @@ __device__ __forceinline__ int compact_problem(const int* __restrict__ order, co
   return order[lo];
 }
 
-// Four one-wave workgroups for each block of the compact grid: 8 of its 32 rows or 2 of its 8 columns.
-__global__ void __launch_bounds__(64, 2) norm_kernel(const oz2_problem* __restrict__ probs,
+// Two workgroups for each block of the compact grid: 16 of its 32 rows or 4 of its 8 columns.
+__global__ void __launch_bounds__(kNormThreads, 2) norm_kernel(const oz2_problem* __restrict__ probs,
                                                   const CrtTables* __restrict__ tab, unsigned long long* __restrict__ cnt,
                                                   const YDesc* __restrict__ yds, const int* __restrict__ order,
                                                   const int* __restrict__ pofs, int nprob) {
   __shared__ NormShared sm;
-  int blk = (int)blockIdx.x >> 2;
-  const int sub = (int)blockIdx.x & 3, pi = compact_problem(order, pofs, nprob, blk);
+  int blk = (int)blockIdx.x >> 1;
+  const int sub = (int)blockIdx.x & 1, pi = compact_problem(order, pofs, nprob, blk);
   const oz2_problem& pr = probs[pi];
   const int N = pr.num_moduli;
   if (N < 1 || N > kMaxModuli || pr.alpha == 0.0) return;
   const int a_blocks = (pr.m + kARows - 1) / kARows;
   int32_t* const nfo = yds ? yds[pi].nf : nullptr;
   int* const nff = yds ? const_cast<int*>(&yds[pi].nff) : nullptr;
-  const int lane = threadIdx.x;
+  const int tid = threadIdx.x;
   if (blk < a_blocks) {
-    const int i = blk * kARows + 8 * sub + (lane & 7);
+    const int i = blk * kARows + kNormRows * sub + (tid & 15);
     const bool valid = i < pr.m;
     const NormOut o{pr.row_shift, pr.m, i, (const GLOBAL double*)pr.A + (valid ? i : 0), (size_t)pr.lda,
                     nfo ? nfo + (size_t)kNfWords * i : nullptr, yds ? yds[pi].fr : nullptr};
-    norm_wave<true>(o, valid, pr.k, tab->T[N], sm, cnt, nff);
+    norm_group<true>(o, valid, pr.k, tab->T[N], sm, cnt, nff);
   } else {
-    const int j = (blk - a_blocks) * kBCols + 2 * sub + (lane >> 5);
+    const int j = (blk - a_blocks) * kBCols + kNormCols * sub + (tid >> 5);
     const bool valid = j < pr.n;
     const NormOut o{pr.col_shift, pr.n, j, (const GLOBAL double*)pr.B + (valid ? (size_t)j * pr.ldb : 0), 1,
                     nfo ? nfo + (size_t)kNfWords * ((size_t)pr.m + j) : nullptr, yds ? yds[pi].fc : nullptr};
-    norm_wave<false>(o, valid, pr.k, tab->T[N], sm, cnt, nff);
+    norm_group<false>(o, valid, pr.k, tab->T[N], sm, cnt, nff);
   }
 }
 
@@ -962,9 +968,9 @@ __global__ void __launch_bounds__(kThreads, 4) residue_kernel(const oz2_problem*
   const bool packed = pr.kp <= packed_kp, rows = blk < a_blocks;
   const int split = (int)blockIdx.y - 1, nsplit = (int)gridDim.y - 1;
   if (split < 0) {
-    const int wave = threadIdx.x >> 6;
-    if (rows) walk_rows(pr, blk * kARows + 8 * wave);
-    else walk_cols(pr, (blk - a_blocks) * kBCols + 2 * wave);
+    __builtin_amdgcn_s_setprio(3);   // few, serial and latency-bound beside the residues' arithmetic
+    if (rows) walk_rows(pr, blk * kARows, sm);
+    else walk_cols(pr, (blk - a_blocks) * kBCols);
   } else if (rows) {
     prep_rows<kWide, true>(pr, tab, blk, split, nsplit, sm, nullptr, N, packed, nullptr, nullptr, false, nullptr, 0);
   } else {
@@ -1048,7 +1054,7 @@ int prep_launch(const oz2_problem* d, int num, int max_m, int max_n, hipStream_t
   const bool wide = !(ht->T[max_moduli] < 0x1.8p62);
   if (launches) *launches = 1;
   if (launches && pofs && fold_q && g_force_split == 0 && prep_two_pass(blocks, elems, c->num_cus)) {
-    hipLaunchKernelGGL(norm_kernel, dim3(4 * (unsigned)blocks), dim3(64), 0, s, d, c->tab, c->counters, yd, order, pofs, num);
+    hipLaunchKernelGGL(norm_kernel, dim3(2 * (unsigned)blocks), dim3(kNormThreads), 0, s, d, c->tab, c->counters, yd, order, pofs, num);
     const unsigned Sr = (unsigned)std::min<long long>(64, (8LL * c->num_cus + blocks - 1) / blocks);
     const dim3 gr((unsigned)blocks, 1 + Sr);
     if (wide)
