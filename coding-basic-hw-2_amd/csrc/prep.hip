@@ -20,7 +20,8 @@
 //   * A (column-major in HBM, row-major residues out): a block owns 32 rows.  The chain threads
 //     load a 32 x 128 k-tile with 256-byte coalesced reads, keep the ordered chain sums, and
 //     park the doubles in LDS k-major; then every thread takes 16 consecutive k of one row,
-//     computes the residues and writes each plane with one 128-bit store.
+//     four lanes to a 64-byte k-block, computes the residues and writes each plane with one
+//     128-bit store.
 //   * B (column-major = K contiguous): 32 lanes per column, 4 consecutive k per lane: 1 KB
 //     coalesced loads, 128 contiguous residue bytes per plane per store.  With two-word digits and
 //     k <= 1024 a column is read once: lane l keeps k = l (mod 32) in registers (its norm chain)
@@ -185,30 +186,27 @@ __device__ __forceinline__ void scaled(const double* x, int sh, double* out) {
     for (int e = 0; e < NE; ++e) out[e] = mul_pow2(x[e], sh);
   }
 }
+template <int NE>
+__device__ __forceinline__ void store_bytes(GLOBAL int8_t* d, const uint32_t* q) {   // NE bytes, one store
+  if constexpr (NE == 16)
+    *(GLOBAL u32x4*)(d) = u32x4{q[0], q[1], q[2], q[3]};
+  else if constexpr (NE == 8)
+    *(GLOBAL u32x2*)(d) = u32x2{q[0], q[1]};
+  else
+    *(GLOBAL uint32_t*)(d) = q[0];
+}
 // Residue planes 0..N-1 of NE consecutive k (integer-valued doubles) of one row / column: NE bytes
-// per plane at dst + l * stride (one 128-bit or 32-bit store).  Three-word digits of 16 values
-// take two passes of 8 (64-bit stores), which keeps the kernel's register count for the common
-// two-word case.
+// per plane at dst + l * stride.
 template <int NE, bool kWide>
 __device__ __forceinline__ void planes(const double* xt, int N, const CrtTables* __restrict__ tab, int widx,
                                        GLOBAL int8_t* dst, size_t stride) {
-  constexpr int P = (kWide && NE > 8) ? 8 : NE;   // values per pass
+  Digits<kWide> x[NE];
 #pragma unroll
-  for (int h = 0; h < NE; h += P) {
-    Digits<kWide> x[P];
-#pragma unroll
-    for (int e = 0; e < P; ++e) x[e] = digits_of<kWide>(xt[h + e]);
-    for (int l = 0; l < N; ++l) {
-      uint32_t q[P / 4];
-      residue_bytes<P, kWide>(x, plane_w<kWide>(tab, l, widx), q);
-      GLOBAL int8_t* d = dst + (size_t)l * stride + h;
-      if constexpr (P == 16)
-        *(GLOBAL u32x4*)(d) = u32x4{q[0], q[1], q[2], q[3]};
-      else if constexpr (P == 8)
-        *(GLOBAL u32x2*)(d) = u32x2{q[0], q[1]};
-      else
-        *(GLOBAL uint32_t*)(d) = q[0];
-    }
+  for (int e = 0; e < NE; ++e) x[e] = digits_of<kWide>(xt[e]);
+  for (int l = 0; l < N; ++l) {
+    uint32_t q[NE / 4];
+    residue_bytes<NE, kWide>(x, plane_w<kWide>(tab, l, widx), q);
+    store_bytes<NE>(dst + (size_t)l * stride, q);
   }
 }
 __device__ __forceinline__ uint32_t abs_u8(double a, int sig) {
@@ -372,7 +370,16 @@ __device__ void prep_rows(const oz2_problem& pr, const CrtTables* __restrict__ t
   //      ordered ||dA||, ||A'|| chain sums (the residue values do not depend on the split)
   const int sh_c = sm.shift[r];
   const bool nf_c = sh_c == OZ2_SHIFT_NONFINITE;
-  const int rr = tid & 31, seg = tid >> 5;   // residue role: row rr, k = 16 seg .. 16 seg + 15
+  // residue role: row rr and W consecutive k, the lanes of a 64-byte k-block of a row side by side, so
+  // that a wave's store of a plane covers whole 64-byte lines (1 KB in a row when the planes are
+  // packed; with lane = row, half-written lines 64 bytes apart: 64 x 1024^3 per call 2571 -> 2540 us,
+  // 2 x 8192^2 x 16384 33.1 -> 32.6 ms, the residues of 2 x 984 x 40000 with 18 moduli 911 -> 745 us).
+  // Two-word digits: 16 k in one pass; three-word ones: 8 k of both halves of the tile.
+  constexpr int W = kWide ? 8 : 16;
+  const int rr = kWide ? tid >> 3 : (tid >> 2) & 31;
+  const int kr = kWide ? 8 * (tid & 7) : 16 * ((tid & 3) + 4 * (tid >> 7));   // + 64 per pass
+  // LDS row of (k, row): the k-segments a wave reads together fall into different banks
+  auto trow = [](int k, int row) { return kWide ? row ^ ((k >> 3) & 3) << 3 : row ^ ((k >> 4) & 1) << 4; };
   const int sh_r = sm.shift[rr], sg_r = sm.sig[rr];
   const bool nf_r = sh_r == OZ2_SHIFT_NONFINITE;
   const bool rvalid = row0 + rr < m;
@@ -406,31 +413,34 @@ __device__ void prep_rows(const oz2_problem& pr, const CrtTables* __restrict__ t
       }
     }
 #pragma unroll
-    for (int jj = 0; jj < kATile / kChains; ++jj) sm.tile[c + kChains * jj][r] = av[jj];
+    for (int jj = 0; jj < kATile / kChains; ++jj) sm.tile[c + kChains * jj][trow(c + kChains * jj, r)] = av[jj];
     __syncthreads();
-    const int kb = k0 + 16 * seg;
-    if (t >= w0 && t < w1 && rvalid && kb < Kp) {
+#pragma unroll
+    for (int h = 0; h < 16 / W; ++h) {
+      const int kl = kr + 64 * h, kb = k0 + kl;
+      if (t < w0 || t >= w1 || !rvalid || kb >= Kp) continue;
       GLOBAL int8_t* dst = (GLOBAL int8_t*)pr.A8 + (packed ? packed_offset(row0 + rr, kb, m, Kp) : (size_t)(row0 + rr) * Kp + kb);
       if (nf_r) {
-        if (zero_nf)
-          for (int l = 0; l <= N; ++l)
-            *(GLOBAL u32x4*)(dst + (size_t)l * pr.a8_mod_stride) = u32x4{0u, 0u, 0u, 0u};
+        if (zero_nf) {
+          const uint32_t zero[4] = {0u, 0u, 0u, 0u};
+          for (int l = 0; l <= N; ++l) store_bytes<W>(dst + (size_t)l * pr.a8_mod_stride, zero);
+        }
       } else {
-        double av[16], xt[16];
+        double av[W], xt[W];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) av[e] = sm.tile[16 * seg + e][rr];
-        uint32_t q[4];   // abs plane first, so the A values are dead during the residue planes
+        for (int e = 0; e < W; ++e) av[e] = sm.tile[kl + e][trow(kl + e, rr)];
+        uint32_t q[W / 4];   // abs plane first, so the A values are dead during the residue planes
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
+        for (int w = 0; w < W / 4; ++w) {
           q[w] = 0u;
 #pragma unroll
           for (int e = 0; e < 4; ++e) q[w] |= abs_u8(av[4 * w + e], sg_r) << (8 * e);
         }
-        *(GLOBAL u32x4*)(dst + (size_t)N * pr.a8_mod_stride) = u32x4{q[0], q[1], q[2], q[3]};
-        scaled<16>(av, sh_r, xt);
+        store_bytes<W>(dst + (size_t)N * pr.a8_mod_stride, q);
+        scaled<W>(av, sh_r, xt);
 #pragma unroll
-        for (int e = 0; e < 16; ++e) xt[e] = trunc(xt[e]);
-        planes<16, kWide>(xt, N, tab, widx, dst, pr.a8_mod_stride);
+        for (int e = 0; e < W; ++e) xt[e] = trunc(xt[e]);
+        planes<W, kWide>(xt, N, tab, widx, dst, pr.a8_mod_stride);
       }
     }
     __syncthreads();
