@@ -1085,20 +1085,23 @@ __global__ void __launch_bounds__(kThreads, 7) dots_kernel(const oz2_problem* __
   // workgroup-uniform: moved to scalar registers, and everything derived from them with them
   const unsigned long long rmask = uniform_u64(rcm[0]), cmask = uniform_u64(rcm[1]);
   const int nR = __popcll(rmask), nC = __popcll(cmask);
-  if (autof && nR * nC <= kCompactMax) {   // workgroup-uniform
-    // dense crossings with enough chains go to the crossings pass, which runs the crossings of all
-    // deferred rows and columns of the problem as one GEMM on the matrix cores (needs the gather
-    // workspace AT)
-    const bool defer = form == kDotFormAuto && yds[pi].AT && total >= kBandMin && 2 * total >= nR * nC;
-    publish(defer);
-    if (defer) {
-      if (t == 0) {
-        unsigned long long* const X = reinterpret_cast<unsigned long long*>(yds[pi].X);
-        atomicOr(&X[r0 >> 6], rmask);
-        atomicOr(&X[((m + 63) >> 6) + (c0 >> 6)], cmask);
-      }
-      return;
+  // Dense crossings with enough chains go to the crossings pass, which runs the crossings of all deferred
+  // rows and columns of the problem as one GEMM on the matrix cores (needs the gather workspace AT) --
+  // however many they are: a tile past the compact form's limit would run them block by block, and
+  // one such tile (17 x 16 finite rows and columns of 2048^3 with 0.1 % NaN / Inf) held the whole pass
+  // for 0.97 ms of 1.36 (16 x 2048^3 + 2 x 2048^2 x 65536).
+  const bool defer = form == kDotFormAuto && yds[pi].AT && total >= kBandMin && 2 * total >= nR * nC;   // workgroup-uniform
+  if (defer) {
+    publish(true);
+    if (t == 0) {
+      unsigned long long* const X = reinterpret_cast<unsigned long long*>(yds[pi].X);
+      atomicOr(&X[r0 >> 6], rmask);
+      atomicOr(&X[((m + 63) >> 6) + (c0 >> 6)], cmask);
     }
+    return;
+  }
+  publish(false);
+  if (autof && nR * nC <= kCompactMax) {   // workgroup-uniform
     if (t < 64) {
       if ((rmask >> t) & 1ull) rmap[__popcll(rmask & ((1ull << t) - 1ull))] = (uint8_t)t;
       if ((cmask >> t) & 1ull) cmap[__popcll(cmask & ((1ull << t) - 1ull))] = (uint8_t)t;
@@ -1107,7 +1110,6 @@ __global__ void __launch_bounds__(kThreads, 7) dots_kernel(const oz2_problem* __
     compact_dots(pr, r0, c0, fl, rmap, cmap, nR, nC, buf);
     return;
   }
-  publish(false);
   const int j = c0 + 16 * w + (lane & 15);
   for (int bi = 0; bi < 4; ++bi) {   // wave w: the blocks (bi, w)
     const int i0 = r0 + 16 * bi + 4 * (lane >> 4);

@@ -1,0 +1,41 @@
+"""The dot pass defers a tile's dense crossings to the crossings pass whatever their number: tiles with
+just under, at and past the compact form's 256 crossings, all uncertified entries repaired, bitwise
+against the oracle with equal counters, and equal to the handle that defers nothing."""
+import numpy as np
+import pytest
+
+import ggemm as G
+import oracle_lib as O
+from gpu_util import same_bits, say
+from test_gpu_grouped import Case, check_case, kernel_handle, run
+
+pytestmark = pytest.mark.gpu
+
+CFG = G.Config(0, 1e-15, 1, G.REPAIR_ON)
+
+
+@pytest.mark.parametrize("rows,cols", [(16, 16), (17, 16), (24, 30), (31, 32)])
+@pytest.mark.parametrize("beta", [0.0, 0.5])
+def test_dense_crossings(rows, cols, beta):
+    say(f"dense crossings {rows} x {cols} per tile, beta {beta}")
+    outs = []
+    for form in ("", "tile"):
+        case = Case([(130, 128, 300), (64, 64, 257)], 91, phi=4.0, beta=beta)
+        rng = np.random.default_rng(3)
+        for h in case.hp:   # all but `rows` rows and `cols` columns of each 64 x 64 tile hold a NaN
+            for r0 in range(0, h.m, 64):
+                for i in rng.permutation(np.arange(r0, min(r0 + 64, h.m)))[rows:]:
+                    h.A[i + 7 * h.lda] = np.nan
+            for c0 in range(0, h.n, 64):
+                for j in rng.permutation(np.arange(c0, min(c0 + 64, h.n)))[cols:]:
+                    h.B[5 + j * h.ldb] = np.nan
+        case.alloc()
+        env = {"GGEMM_DOT_FORM": form} if form else {}
+        with kernel_handle(case, None, GGEMM_STATS_REPAIR="1", **env) as hd:
+            rc, st = run(case, G.PATH_EMU_GROUPED, CFG, handle=hd)
+        assert rc == 0
+        check_case(case, G.PATH_EMU_GROUPED, CFG, st, O.REPAIR_ON)
+        assert st.num_repaired >= 0.5 * rows * cols
+        outs.append([case.C(g).copy() for g in range(2)])
+    for a, b in zip(*outs):
+        assert same_bits(a, b)
