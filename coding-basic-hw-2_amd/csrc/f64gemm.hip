@@ -237,39 +237,48 @@ __global__ void __launch_bounds__(kThreads, OCC) f64_grouped_kernel(const F64Pro
   // With beta != 0 the C0 values of a batch of blocks are all loaded before the batch's stores:
   // entry by entry, each C0 load waited for its data before the store (the stores might alias
   // the next loads), one memory round trip per entry.
+  // C0 rows and columns past the problem are read from its last one, so the loads need no test.  The
+  // product by alpha is rounded, the one by beta fused, at every shape.
   const size_t ldc = (size_t)P.ldc;
   GLOBAL double* const Cg = (GLOBAL double*)P.C;
   const bool rd = P.beta != 0.0;
   constexpr int NBLK = FM * FN, BATCH = NBLK < 8 ? NBLK : 8;
+  auto epilogue = [&](auto inside) {
+    constexpr bool kInside = decltype(inside)::value;   // the whole tile
 #pragma unroll
-  for (int b0 = 0; b0 < NBLK; b0 += BATCH) {
-    double c0[BATCH][4];
+    for (int b0 = 0; b0 < NBLK; b0 += BATCH) {
+      double c0[BATCH][4];
+      if (rd) {
 #pragma unroll
-    for (int q = 0; q < BATCH; ++q) {
-      const int i = (b0 + q) / FN, j = (b0 + q) % FN;
-      const int row = row0 + (WM * i + wm) * 16 + (lane & 15);
-      const int cbase = col0 + (WN * j + wn) * 16 + (lane >> 4);
+        for (int q = 0; q < BATCH; ++q) {
+          const int i = (b0 + q) / FN, j = (b0 + q) % FN;
+          const int row = row0 + (WM * i + wm) * 16 + (lane & 15), rc = kInside ? row : min(row, P.m - 1);
+          const int cbase = col0 + (WN * j + wn) * 16 + (lane >> 4);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int col = cbase + 4 * r;
-        c0[q][r] = (rd && row < P.m && col < P.n) ? Cg[(size_t)row + (size_t)col * ldc] : 0.0;
+          for (int r = 0; r < 4; ++r)
+            c0[q][r] = Cg[(size_t)rc + (size_t)(kInside ? cbase + 4 * r : min(cbase + 4 * r, P.n - 1)) * ldc];
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < BATCH; ++q) {
+        const int i = (b0 + q) / FN, j = (b0 + q) % FN;
+        const int row = row0 + (WM * i + wm) * 16 + (lane & 15);
+        const int cbase = col0 + (WN * j + wn) * 16 + (lane >> 4);
+        if (!kInside && row >= P.m) continue;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int col = cbase + 4 * r;
+          if (!kInside && col >= P.n) continue;
+          const double ab = compute ? P.alpha * acc[i][j][r] : 0.0;
+          Cg[(size_t)row + (size_t)col * ldc] = !rd ? ab : (compute ? __builtin_fma(P.beta, c0[q][r], ab) : P.beta * c0[q][r]);
+        }
       }
     }
-#pragma unroll
-    for (int q = 0; q < BATCH; ++q) {
-      const int i = (b0 + q) / FN, j = (b0 + q) % FN;
-      const int row = row0 + (WM * i + wm) * 16 + (lane & 15);
-      const int cbase = col0 + (WN * j + wn) * 16 + (lane >> 4);
-      if (row >= P.m) continue;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int col = cbase + 4 * r;
-        if (col >= P.n) continue;
-        const double ab = compute ? P.alpha * acc[i][j][r] : 0.0;
-        Cg[(size_t)row + (size_t)col * ldc] = !rd ? ab : (compute ? ab + P.beta * c0[q][r] : P.beta * c0[q][r]);
-      }
-    }
-  }
+  };
+  if (row0 + BM <= P.m && col0 + BN <= P.n)
+    epilogue(std::true_type{});
+  else
+    epilogue(std::false_type{});
 }
 
 // Few outputs (32 x 32 tiles, 512 threads, one workgroup per compute unit): waves 0-3 run one
@@ -346,7 +355,7 @@ __global__ void __launch_bounds__(2 * kThreads, 2) f64_chain_kernel(const F64Pro
   for (int r = 0; r < 4; ++r) {
     if (cbase + 4 * r >= P.n) continue;
     const double ab = compute ? P.alpha * acc[r] : 0.0;
-    Cg[(size_t)row + (size_t)(cbase + 4 * r) * ldc] = !rd ? ab : (compute ? ab + P.beta * c0[r] : P.beta * c0[r]);
+    Cg[(size_t)row + (size_t)(cbase + 4 * r) * ldc] = !rd ? ab : (compute ? __builtin_fma(P.beta, c0[r], ab) : P.beta * c0[r]);
   }
 }
 
