@@ -303,6 +303,15 @@ __device__ void prep_rows(const oz2_problem& pr, const CrtTables* __restrict__ t
   #pragma unroll
         for (int t = 0; t < 16; ++t) step(a[t], k0 + 8 * t);
       };
+      // a row that holds a NaN is read no further (trk): its shift is non-finite and each of its entries
+      // NaN, whatever follows (16 x 2048^3 + 2 x 2048^2 x 65536 with 0.1 % NaN / Inf: 3.39 -> 2.68 ms
+      // per call; finite groups the same)
+      bool nan = false;
+      auto nan_row = [&]() {
+        if (!trk) return false;
+        if (isnan(ss)) sm.nfnan[r] = 1;
+        return *(volatile int*)&sm.nfnan[r] != 0;
+      };
       if (k + 8 * 15 < K) {
         double a[16], b[16];
         ld16(a, k);
@@ -316,10 +325,12 @@ __device__ void prep_rows(const oz2_problem& pr, const CrtTables* __restrict__ t
           ld16(a, more ? k + 128 : k);
           chain16(b, k);
           k += 128;
-          if (!more) break;
+          nan = nan_row();
+          if (!more || nan) break;
         }
       }
-      for (; k < K; k += 8) step(A[i + (size_t)k * lda], k);
+      if (!nan)
+        for (; k < K; k += 8) step(A[i + (size_t)k * lda], k);
       if (trk && isnan(ss)) sm.nfnan[r] = 1;   // a sum of squares turns NaN only through a NaN
     }
     sm.red0[c][r] = mx;
@@ -570,6 +581,7 @@ __device__ void prep_cols(const oz2_problem& pr, const CrtTables* __restrict__ t
 #pragma unroll
       for (int t = 0; t < 16; ++t) step(a[t], k0 + 32 * t);
     };
+    bool nan = false;   // as for the A rows
     if (k + 32 * 15 < K) {
       double a[16], c[16];
       ld16(a, k);
@@ -583,10 +595,12 @@ __device__ void prep_cols(const oz2_problem& pr, const CrtTables* __restrict__ t
         ld16(a, more ? k + 512 : k);
         chain16(c, k);
         k += 512;
-        if (!more) break;
+        nan = trk && (uint32_t)(__ballot(isnan(ss)) >> (threadIdx.x & 32)) != 0u;   // any lane of the column
+        if (!more || nan) break;
       }
     }
-    for (; k < K; k += 32) step(b[k], k);
+    if (!nan)
+      for (; k < K; k += 32) step(b[k], k);
   }
   if (trk && isnan(ss)) sm.nfnan[w] = 1;   // a sum of squares turns NaN only through a NaN
 #pragma unroll
