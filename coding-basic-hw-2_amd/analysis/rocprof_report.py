@@ -43,7 +43,7 @@ FP64_PEAK = 78.6e12    # MI355X dense FP64 MFMA, flop / s
 
 STAGES = ("prep", "i8_gemm", "reconstruct", "native", "memops")
 _STAGE_RE = [
-    (re.compile(r"\bprep_kernel\b"), "prep"),
+    (re.compile(r"\b(prep|norm|residue)_kernel\b"), "prep"),
     (re.compile(r"\bi8_(grouped|large)(_persistent)?_kernel\b"), "i8_gemm"),
     (re.compile(r"\b(recon|dots|gather|cross)_kernel\b"), "reconstruct"),
     (re.compile(r"\bf64_\w*kernel\b"), "native"),

@@ -4,9 +4,9 @@
 // scratch are allocated in ggemm_create_ex; a call validates, plans, writes every descriptor into
 // a double-buffered pinned slot, issues ONE H2D of the used part of the blob and then the
 // kernels: prep -> grouped INT8 GEMM -> reconstruct -> FP64 dot products of the entries the
-// reconstruct flagged (4 launches for any group size; 3 when the digits are column-major, where the
-// reconstruct computes them itself) plus one grouped native FP64 GEMM launch when some problems
-// take a native route.
+// reconstruct flagged (six launches for any group size, one more when prep takes two; three when the
+// digits are column-major, where the reconstruct computes the dot products itself) plus one grouped
+// native FP64 GEMM launch when some problems take a native route.
 #include <algorithm>
 #include <cmath>
 #include <cstddef>

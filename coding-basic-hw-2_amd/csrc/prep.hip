@@ -1,4 +1,5 @@
-// prep.hip -- Ozaki-II residue preparation for a whole group (one launch).
+// prep.hip -- Ozaki-II residue preparation for a whole group (one launch; two for few rows and columns
+// over a long k, below).
 //
 // Per problem (alpha != 0, N moduli):
 //   s_i   = largest s with 2^s ||A(i,:)||_2 (1+2^-30)^(1/2) <= T_N   (t_j likewise for B(:,j))
