@@ -244,8 +244,8 @@ constexpr int kPrepRows = 32, kPrepCols = 8;
 // launch word for f64_launch: the tile count in bits 0-27, the tile shape from bit kF64ShapeBit (0:
 // nothing to launch).  tile_mode 0 chooses the shape from the group's problems, 64 or 128 forces square
 // tiles of that edge.
-enum {   // 64 x 64, 128 x 128, 16 x 128, 32 x 128, 32 x 32 with one accumulator chain per wave
-  kF64Tile64 = 0, kF64Tile128 = 1, kF64Tile16 = 2, kF64Tile32 = 3, kF64TileChain = 4, kF64Shapes = 5
+enum {   // 64 x 64, 128 x 128, 16 x 128, 32 x 128, 32 x 32 with one accumulator chain per wave (128- / 64-deep stages)
+  kF64Tile64 = 0, kF64Tile128 = 1, kF64Tile16 = 2, kF64Tile32 = 3, kF64TileChain = 4, kF64TileShort = 5, kF64Shapes = 6
 };
 constexpr int kF64ShapeBit = 28, kF64MaxTiles = (1 << kF64ShapeBit) - 1;
 int f64_build_schedule(const F64Problem* h, int num, void* h_ws, size_t ws_bytes, int* launch, size_t* bytes_used,

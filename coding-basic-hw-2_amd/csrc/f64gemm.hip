@@ -281,15 +281,16 @@ __global__ void __launch_bounds__(kThreads, OCC) f64_grouped_kernel(const F64Pro
     epilogue(std::false_type{});
 }
 
-// Few outputs (32 x 32 tiles, 512 threads, one workgroup per compute unit): waves 0-3 run one
+// Few outputs (32 x 32 tiles, 512 threads): waves 0-3 run one
 // accumulator chain each -- 16 x 16 outputs, the whole k -- and waves 4-7, one beside each on its SIMD,
-// stream the operands in 128-deep stages, two stages ahead in registers.  A chain takes an MFMA every
+// stream the operands in stages of BK k, two stages ahead in registers.  A chain takes an MFMA every
 // 64-odd cycles whatever else happens, so the time is k / 4 of them as long as the compute waves issue
 // nothing but fragment reads and MFMAs.
-constexpr int kChainTile = 32, kChainBK = 128;
+constexpr int kChainTile = 32;
+template <int BK>
 __global__ void __launch_bounds__(2 * kThreads, 2) f64_chain_kernel(const F64Problem* __restrict__ probs,
                                                                   const int* __restrict__ sched) {
-  constexpr int T = kChainTile, BK = kChainBK;
+  constexpr int T = kChainTile;
   __shared__ double sA[2][BK][T];
   __shared__ __align__(16) double sB[2][BK * T];
   const TileRef t = find_tile(sched, blockIdx.x);
@@ -363,7 +364,7 @@ constexpr int kCus = 256;
 struct F64Shape {
   int bm, bn;
 };
-constexpr F64Shape kShapes[kF64Shapes] = {{64, 64}, {128, 128}, {16, 128}, {32, 128}, {32, 32}};
+constexpr F64Shape kShapes[kF64Shapes] = {{64, 64}, {128, 128}, {16, 128}, {32, 128}, {32, 32}, {32, 32}};
 
 long long tiles_of(const F64Problem& p, const F64Shape& t) {
   return (long long)((p.m + t.bm - 1) / t.bm) * ((p.n + t.bn - 1) / t.bn);
@@ -421,6 +422,10 @@ int f64_build_schedule(const F64Problem* h, int num, void* h_ws, size_t ws_bytes
       if (share >= 0.87 * (full + (left <= 0.0 ? 0.0 : left <= 0.5 ? 0.5 : 1.0))) shape = kF64Tile128;
     }
   }
+  // 32 x 32 tiles: 128-deep stages, one workgroup per compute unit, or 64-deep ones and two of them, when
+  // there is more than a tile for each (3 x 300x300x4096: 106 -> 91 us) or k is too short for the long
+  // stages' start-up (3 x 300x300x100 19.2 -> 14.8; 500x500x512 18, 500x500x4096 58 against 64 us)
+  if (shape == kF64TileChain && (tiles[kF64TileChain] > kCus || kmax <= 512)) shape = kF64TileShort;
   const F64Shape& t = kShapes[shape];
   long long tot = 0;
   bool equal = true;
@@ -447,8 +452,9 @@ int f64_launch(const F64Problem* d_probs, const void* d_sched, int launch, hipSt
   const unsigned tiles = (unsigned)(launch & kF64MaxTiles);
   const int shape = launch >> kF64ShapeBit;
   const int* sched = static_cast<const int*>(d_sched);
-  if (shape == kF64TileChain) {
-    hipLaunchKernelGGL(f64_chain_kernel, dim3(tiles), dim3(2 * kThreads), 0, s, d_probs, sched);
+  if (shape == kF64TileChain || shape == kF64TileShort) {
+    const auto kernel = shape == kF64TileChain ? f64_chain_kernel<128> : f64_chain_kernel<64>;
+    hipLaunchKernelGGL(kernel, dim3(tiles), dim3(2 * kThreads), 0, s, d_probs, sched);
   } else {
     const auto kernel = shape == kF64Tile128  ? f64_grouped_kernel<128, 128, 2, 2>
                         : shape == kF64Tile16 ? f64_grouped_kernel<16, 128, 1, 4>

@@ -17,6 +17,8 @@ GROUPS = {
     "chain_edges": [(32, 32, 128), (33, 31, 127), (31, 33, 129), (64, 1, 255), (1, 64, 256), (70, 50, 257), (1, 1, 1),
                     (40, 40, 0), (0, 5, 5), (48, 48, 385)],
     "chain_long_k": [(70, 50, 9000), (65, 1, 8191), (5, 40, 12345)],
+    "chain_513": [(64, 60, 513), (31, 32, 512), (33, 1, 640)],     # 128-deep stages from k = 513
+    "chain_257_tiles": [(32 * 16, 32 * 16, 700), (20, 20, 650)],   # 64-deep ones past 256 tiles
     "chain_alpha0": [(50, 40, 300, 0.0, 0.5), (50, 40, 300, -1.0, 0.0)],
     # enough thin problems for the thin tiles
     "thin16": [(1 + i % 16, 120 + i % 20, 1 + i % 50) for i in range(300)],
