@@ -333,7 +333,9 @@ __global__ void __launch_bounds__(2 * kThreads, 2) f64_chain_kernel(const F64Pro
     __builtin_amdgcn_s_setprio(3);
     __syncthreads();
     for (int kt = 0; kt < nk; ++kt) {
-      const int steps = (P.k - kt * BK + 3) / 4;   // the steps past k would add zeros
+      // the last 16-deep k group whole, as at every other shape: its zeros past k turn a chain of -0 (negative
+      // products that underflow) into +0, so the shapes would differ in that sign if one left them out
+      const int steps = (P.k - kt * BK + kBK - 1) / kBK * (kBK / 4);
       if (steps >= BK / 4) {
 #pragma unroll
         for (int s = 0; s < BK / 4; ++s) step(kt & 1, s);

@@ -3,6 +3,7 @@ rule that chooses: 32 x 32 tiles (few outputs), 16 x 128 and 32 x 128 tiles (man
 128 x 128 tiles (filled rounds).  Every shape takes the same k-ordered chain per entry, so each result
 equals the 64 x 64 kernel's (forced with GGEMM_F64_TILE) bit for bit; that kernel is held to the
 componentwise gamma_n bound against the host's extended-precision dots."""
+import numpy as np
 import pytest
 
 import ggemm as G
@@ -47,3 +48,30 @@ def test_native_shapes(name, beta):
         h.reference()
         gate, _ = h.gate(outs[0][g])
         assert gate <= 1.0, (g, gate)
+
+
+UNDERFLOW = {   # every product underflows to -0: the sign of the result tells how far the chain is padded
+    "short": [(20, 20, k) for k in (1, 4, 8, 12, 15, 16, 20, 60, 64, 68, 130)],
+    "chain": [(20, 20, k) for k in (4, 16, 600, 624, 1020, 1032)],
+    "thin16": [(1 + i % 16, 130, 4 + i % 17) for i in range(300)],
+    "thin32": [(17 + i % 16, 250, 4 + i % 17) for i in range(300)],
+}
+
+
+@pytest.mark.parametrize("name", sorted(UNDERFLOW))
+def test_underflow_sign(name):
+    say(f"underflow: {name}")
+    outs = []
+    for env in ({}, {"GGEMM_F64_TILE": "64"}, {"GGEMM_F64_TILE": "128"}):
+        case = Case(UNDERFLOW[name], 5)
+        for h in case.hp:
+            h.A[:], h.B[:] = 1e-200, -1e-200
+        case.alloc()
+        with kernel_handle(case, None, **env) as hd:
+            rc, _ = run(case, G.PATH_NATIVE_GROUPED, CFG, handle=hd)
+        assert rc == 0
+        outs.append([case.C(g).copy() for g in range(len(case.hp))])
+    for g, h in enumerate(case.hp):
+        assert np.array_equal(outs[1][g], np.zeros(h.m * h.n))
+        assert np.signbit(outs[1][g]).all() == (h.k % 16 == 0)   # +0 once the chain is padded past k
+        assert same_bits(outs[0][g], outs[1][g]) and same_bits(outs[2][g], outs[1][g]), (g, UNDERFLOW[name][g])
