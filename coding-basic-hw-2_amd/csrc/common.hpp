@@ -77,6 +77,9 @@ struct F64Problem {
   double alpha, beta;
 };
 
+// ceil(x / b) for every x >= 0: x + b - 1 would wrap for the largest b - 1 sizes an int holds
+__host__ __device__ constexpr int ceil_div(int x, int b) { return x / b + (x % b != 0); }
+
 // Schedule image shared by the tile-based kernels (INT8 GEMM, FP64 GEMM):
 //   int[0] total tiles, int[1] entries, int[2] tiles per entry when all entries have the same
 //   count (INT8 GEMM; 0 otherwise), int[3] the persistent queues' chunk, int[kHdrHw] the units the

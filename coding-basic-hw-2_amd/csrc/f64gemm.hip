@@ -119,7 +119,7 @@ struct Loader {
   }
   __device__ __forceinline__ void load(Regs& r, int kt) const {
     const int k0 = kt * BK;
-    if (k0 + BK <= k) {
+    if (k - k0 >= BK) {
       const GLOBAL double* pa = Ag + (size_t)(k0 + ak) * lda;
 #pragma unroll
       for (int q = 0; q < NA; ++q) r.a[q] = pa[(size_t)(KSA * q) * lda];
@@ -164,13 +164,13 @@ __global__ void __launch_bounds__(kThreads, OCC) f64_grouped_kernel(const F64Pro
   const TileRef t = find_tile(sched, blockIdx.x);
   const F64Problem P = probs[t.problem];
   const int local = t.local;
-  const int tiles_m = (P.m + BM - 1) / BM;
+  const int tiles_m = ceil_div(P.m, BM);
   const int row0 = (local % tiles_m) * BM, col0 = (local / tiles_m) * BN;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % WM, wn = wave / WM;
   // this wave's blocks inside the problem: block i covers rows row0 + 16 (WM i + wm) ..
-  const int nbm = min(FM, max(0, (P.m - row0 - 16 * wm + 16 * WM - 1) / (16 * WM)));
-  const int nbn = min(FN, max(0, (P.n - col0 - 16 * wn + 16 * WN - 1) / (16 * WN)));
+  const int nbm = min(FM, ceil_div(max(0, P.m - row0 - 16 * wm), 16 * WM));
+  const int nbn = min(FN, ceil_div(max(0, P.n - col0 - 16 * wn), 16 * WN));
 
   v4d acc[FM][FN];
 #pragma unroll
@@ -182,7 +182,7 @@ __global__ void __launch_bounds__(kThreads, OCC) f64_grouped_kernel(const F64Pro
   if (compute) {
     Loader<BM, BN, BK> ld;
     ld.init(P, row0, col0, tid);
-    const int nk = (P.k + BK - 1) / BK;
+    const int nk = ceil_div(P.k, BK);
     const int fr = lane & 15, fk = lane >> 4;
     // The product is taken transposed (B's columns as the MFMA rows), so that a lane's four results
     // are four columns of one row and 16 lanes store 16 consecutive rows of a column: 128-byte
@@ -275,7 +275,7 @@ __global__ void __launch_bounds__(kThreads, OCC) f64_grouped_kernel(const F64Pro
       }
     }
   };
-  if (row0 + BM <= P.m && col0 + BN <= P.n)
+  if (P.m - row0 >= BM && P.n - col0 >= BN)
     epilogue(std::true_type{});
   else
     epilogue(std::false_type{});
@@ -295,11 +295,11 @@ __global__ void __launch_bounds__(2 * kThreads, 2) f64_chain_kernel(const F64Pro
   __shared__ __align__(16) double sB[2][BK * T];
   const TileRef t = find_tile(sched, blockIdx.x);
   const F64Problem P = probs[t.problem];
-  const int tiles_m = (P.m + T - 1) / T;
+  const int tiles_m = ceil_div(P.m, T);
   const int row0 = (t.local % tiles_m) * T, col0 = (t.local / tiles_m) * T;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool compute = P.alpha != 0.0 && P.k > 0;
-  const int nk = compute ? (P.k + BK - 1) / BK : 0;
+  const int nk = compute ? ceil_div(P.k, BK) : 0;
   if (wave >= 4) {
     if (!compute) return;
     Loader<T, T, BK> ld;
@@ -335,7 +335,7 @@ __global__ void __launch_bounds__(2 * kThreads, 2) f64_chain_kernel(const F64Pro
     for (int kt = 0; kt < nk; ++kt) {
       // the last 16-deep k group whole, as at every other shape: its zeros past k turn a chain of -0 (negative
       // products that underflow) into +0, so the shapes would differ in that sign if one left them out
-      const int steps = (P.k - kt * BK + kBK - 1) / kBK * (kBK / 4);
+      const int steps = ceil_div(P.k - kt * BK, kBK) * (kBK / 4);
       if (steps >= BK / 4) {
 #pragma unroll
         for (int s = 0; s < BK / 4; ++s) step(kt & 1, s);
@@ -369,7 +369,7 @@ struct F64Shape {
 constexpr F64Shape kShapes[kF64Shapes] = {{64, 64}, {128, 128}, {16, 128}, {32, 128}, {32, 32}, {32, 32}};
 
 long long tiles_of(const F64Problem& p, const F64Shape& t) {
-  return (long long)((p.m + t.bm - 1) / t.bm) * ((p.n + t.bn - 1) / t.bn);
+  return (long long)ceil_div(p.m, t.bm) * ceil_div(p.n, t.bn);
 }
 
 }  // namespace
