@@ -413,10 +413,12 @@ int f64_build_schedule(const F64Problem* h, int num, void* h_ws, size_t ws_bytes
   int shape = tile_mode == 128 ? kF64Tile128 : kF64Tile64;
   if (tile_mode == 0 && kmax > 0) {
     auto rounds = [&](int s) { return std::ceil((double)tiles[s] / kCus); };
+    // a grid has fewer than 2^32 threads: the 32 x 32 tiles, twice the threads each, are refused first
+    const bool small = tiles[kF64TileChain] < (1LL << 32) / (2 * kThreads);
     if (mmax <= 32) {
       const int thin = mmax <= 16 ? kF64Tile16 : kF64Tile32;
-      shape = 0.4 * rounds(kF64TileChain) < std::max(1.2, 1.0 * rounds(thin)) ? kF64TileChain : thin;
-    } else if (0.22 * rounds(kF64TileChain) < std::max(0.85, 0.58 * rounds(kF64Tile64))) {
+      shape = small && 0.4 * rounds(kF64TileChain) < std::max(1.2, 1.0 * rounds(thin)) ? kF64TileChain : thin;
+    } else if (small && 0.22 * rounds(kF64TileChain) < std::max(0.85, 0.58 * rounds(kF64Tile64))) {
       shape = kF64TileChain;
     } else if (area >= 0.95 * 16384.0 * tiles[kF64Tile128]) {
       const double share = work128 / kmax / (2.0 * kCus);

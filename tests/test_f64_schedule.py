@@ -49,6 +49,17 @@ def test_largest_sizes(n):
         assert tiles == ceil(shape[0], TILE[tile][0]) * ceil(shape[1], TILE[tile][1]), shape
 
 
+@pytest.mark.parametrize("group", [[(2 ** 28, 1, 300)], [(2 ** 29, 16, 300)], [(2 ** 28 - 32, 1, 300)],
+                                   [(5, 33, 300)] * 40 + [(30, 2 ** 27, 300), (31, 2 ** 27, 300)]])
+def test_grid_limit(group):
+    """A grid of 2^32 threads is refused by the runtime: whatever 64 x 64 tiles could run, the chosen
+    shape can."""
+    rc, tile, tiles, _ = schedule(group)
+    assert rc == 0
+    assert sum(ceil(m, 64) * ceil(n, 64) for m, n, _ in group) * 256 < 2 ** 32
+    assert tiles * (512 if tile in (CHAIN, SHORT) else 256) < 2 ** 32, (tile, tiles)
+
+
 def test_ceil_div(tmp_path):
     """The division that the kernels take their stages, tiles and blocks from."""
     src = tmp_path / "t.cpp"
