@@ -410,6 +410,8 @@ int f64_build_schedule(const F64Problem* h, int num, void* h_ws, size_t ws_bytes
   // (67 TFLOP/s on long k against 61 of the 64 x 64 tiles) when little of the tiles hangs over the
   // problems' edges and their rounds of two workgroups per compute unit are nearly filled: a short last
   // round leaves compute units idle for as long as a full one, unless it has at most one tile for each.
+  // At most one tile per compute unit in all stays on 64 x 64 tiles, four workgroups of which hide each
+  // other's waits: 2048^2 x 2048 323 against 297 us, x 64 23.9 / 21.4, 16 x 512^3 91 / 84.
   int shape = tile_mode == 128 ? kF64Tile128 : kF64Tile64;
   if (tile_mode == 0 && kmax > 0) {
     auto rounds = [&](int s) { return std::ceil((double)tiles[s] / kCus); };
@@ -423,7 +425,7 @@ int f64_build_schedule(const F64Problem* h, int num, void* h_ws, size_t ws_bytes
     } else if (area >= 0.95 * 16384.0 * tiles[kF64Tile128]) {
       const double share = work128 / kmax / (2.0 * kCus);
       const double full = std::floor(share), left = share - full;
-      if (share >= 0.87 * (full + (left <= 0.0 ? 0.0 : left <= 0.5 ? 0.5 : 1.0))) shape = kF64Tile128;
+      if (share >= 0.87 * (full + (left <= 0.0 ? 0.0 : left <= 0.5 && full > 0.0 ? 0.5 : 1.0))) shape = kF64Tile128;
     }
   }
   // 32 x 32 tiles: 128-deep stages, one workgroup per compute unit, or 64-deep ones and two of them, when

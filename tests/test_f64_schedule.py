@@ -60,6 +60,15 @@ def test_grid_limit(group):
     assert tiles * (512 if tile in (CHAIN, SHORT) else 256) < 2 ** 32, (tile, tiles)
 
 
+@pytest.mark.parametrize("group,tile", [
+    ([(2048, 2048, 64)], T64), ([(2048, 2048, 4096)], T64), ([(1920, 1920, 512)], T64), ([(512, 512, 512)] * 16, T64),
+    ([(1024, 1024, 1500)] * 4, T64), ([(512, 512, 512)] * 32, T128), ([(4096, 4096, 512)], T128),
+    ([(1024, 1024, 1500)] * 12, T128), ([(2816, 2816, 512)], T128), ([(1664, 2048, 512)], T64)])
+def test_128_tiles_fill_a_round(group, tile):
+    """128 x 128 tiles only from a whole round on (two workgroups per compute unit)."""
+    assert schedule(group)[:2] == (0, tile)
+
+
 def test_ceil_div(tmp_path):
     """The division that the kernels take their stages, tiles and blocks from."""
     src = tmp_path / "t.cpp"

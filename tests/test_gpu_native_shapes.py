@@ -24,8 +24,8 @@ GROUPS = {
     # enough thin problems for the thin tiles
     "thin16": [(1 + i % 16, 120 + i % 20, 1 + i % 50) for i in range(300)],
     "thin32": [(1 + i % 32, 250 + i % 9, 15 + i % 35) for i in range(300)],
-    # one full round of 128 x 128 tiles per compute unit and no edges
-    "tile128": [(2048, 2048, 40)],
+    # one full round of 128 x 128 tiles (two per compute unit) and no edges
+    "tile128": [(4096, 2048, 40)],
 }
 
 
