@@ -387,7 +387,7 @@ int f64_build_schedule(const F64Problem* h, int num, void* h_ws, size_t ws_bytes
   int* entry = prefix + ne + 1;
   int mmax = 0, kmax = 0;
   long long tiles[kF64Shapes] = {};
-  double work128 = 0, area = 0;
+  double work128 = 0, workc = 0, area = 0;
   for (int i = 0, j = 0; i < num; ++i) {
     const F64Problem& p = h[i];
     if (p.m <= 0 || p.n <= 0) continue;
@@ -397,6 +397,7 @@ int f64_build_schedule(const F64Problem* h, int num, void* h_ws, size_t ws_bytes
     kmax = std::max(kmax, k);
     for (int s = 0; s < kF64Shapes; ++s) tiles[s] += tiles_of(p, kShapes[s]);
     work128 += (double)tiles_of(p, kShapes[kF64Tile128]) * k;
+    workc += (double)tiles_of(p, kShapes[kF64TileChain]) * k;
     area += (double)p.m * p.n;
   }
   std::sort(entry, entry + ne, [h](int a, int b) {
@@ -415,12 +416,19 @@ int f64_build_schedule(const F64Problem* h, int num, void* h_ws, size_t ws_bytes
   int shape = tile_mode == 128 ? kF64Tile128 : kF64Tile64;
   if (tile_mode == 0 && kmax > 0) {
     auto rounds = [&](int s) { return std::ceil((double)tiles[s] / kCus); };
-    // a grid has fewer than 2^32 threads: the 32 x 32 tiles, twice the threads each, are refused first
-    const bool small = tiles[kF64TileChain] < (1LL << 32) / (2 * kThreads);
+    // 32 x 32 tiles: a grid has fewer than 2^32 threads, and these tiles take twice as many each.  Past the
+    // two workgroups per compute unit that run at once, each further round costs about 1 us before its first
+    // MFMA, which only a longer k makes up for -- 32 (mean over the tiles) for each round, 384 whatever the
+    // rounds.  Below the line, us at 32 x 32 against the shape taken: 2000 x 8x8x16 16.8 / 13.4,
+    // 1000 x 30x60x128 33.8 / 24.6, 600 x 96x96x16 43 / 21, 300 x 96x96x300 71 / 68; above: 71 x 96x96x128
+    // 16.0 / 19.1, 222 x 96x96x256 40.5 / 46.2, 300 x 96x96x400 70 / 82, 5000 x 32x32x400 210 / 217.
+    const double crounds = rounds(kF64TileChain);
+    const bool small = tiles[kF64TileChain] < (1LL << 32) / (2 * kThreads) &&
+                       (crounds <= 2.0 || workc >= std::min(32.0 * crounds, 384.0) * tiles[kF64TileChain]);
     if (mmax <= 32) {
       const int thin = mmax <= 16 ? kF64Tile16 : kF64Tile32;
-      shape = small && 0.4 * rounds(kF64TileChain) < std::max(1.2, 1.0 * rounds(thin)) ? kF64TileChain : thin;
-    } else if (small && 0.22 * rounds(kF64TileChain) < std::max(0.85, 0.58 * rounds(kF64Tile64))) {
+      shape = small && 0.4 * crounds < std::max(1.2, 1.0 * rounds(thin)) ? kF64TileChain : thin;
+    } else if (small && 0.22 * crounds < std::max(0.85, 0.58 * rounds(kF64Tile64))) {
       shape = kF64TileChain;
     } else if (area >= 0.95 * 16384.0 * tiles[kF64Tile128]) {
       const double share = work128 / kmax / (2.0 * kCus);

@@ -69,6 +69,16 @@ def test_128_tiles_fill_a_round(group, tile):
     assert schedule(group)[:2] == (0, tile)
 
 
+@pytest.mark.parametrize("group,tile", [
+    ([(8, 8, 16)] * 512, SHORT), ([(8, 8, 16)] * 513, T16), ([(8, 8, 383)] * 5000, T16), ([(8, 8, 384)] * 5000, SHORT),
+    ([(30, 30, 100)] * 5000, T32), ([(32, 32, 400)] * 5000, SHORT), ([(96, 96, 16)] * 56, SHORT), ([(96, 96, 16)] * 57, T64),
+    ([(96, 96, 95)] * 57, T64), ([(96, 96, 96)] * 57, SHORT), ([(96, 96, 255)] * 222, T64), ([(96, 96, 256)] * 222, SHORT),
+    ([(2 ** 20, 1, 8)], T64), ([(8, 8, 8)] * 5000 + [(8, 8, 1000)], T16), ([(500, 500, 9000)] + [(30, 30, 64)] * 300, SHORT)])
+def test_short_k_rounds(group, tile):
+    """More 32 x 32 tiles than run at once only from a k on that makes up for the start of each round."""
+    assert schedule(group)[:2] == (0, tile)
+
+
 def test_ceil_div(tmp_path):
     """The division that the kernels take their stages, tiles and blocks from."""
     src = tmp_path / "t.cpp"
