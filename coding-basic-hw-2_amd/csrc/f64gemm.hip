@@ -333,18 +333,19 @@ __global__ void __launch_bounds__(2 * kThreads, 2) f64_chain_kernel(const F64Pro
     __builtin_amdgcn_s_setprio(3);
     __syncthreads();
     for (int kt = 0; kt < nk; ++kt) {
-      // the last 16-deep k group whole, as at every other shape: its zeros past k turn a chain of -0 (negative
-      // products that underflow) into +0, so the shapes would differ in that sign if one left them out
-      const int steps = ceil_div(P.k - kt * BK, kBK) * (kBK / 4);
-      if (steps >= BK / 4) {
+      const int left = P.k - kt * BK;
+      if (left > BK - 4) {
 #pragma unroll
         for (int s = 0; s < BK / 4; ++s) step(kt & 1, s);
       } else {
 #pragma unroll 4
-        for (int s = 0; s < steps; ++s) step(kt & 1, s);
+        for (int s = 0; 4 * s < left; ++s) step(kt & 1, s);
       }
       __syncthreads();
     }
+    // the other shapes run zeros up to a multiple of 16 k; all they can change is a chain of -0 (negative
+    // products that underflow), which the +0 of a padded step turns into +0
+    if (P.k % kBK != 0 && P.k % kBK <= kBK - 4) acc = acc + v4d{0.0, 0.0, 0.0, 0.0};
   }
   const size_t ldc = (size_t)P.ldc;
   GLOBAL double* const Cg = (GLOBAL double*)P.C;
