@@ -79,6 +79,29 @@ def test_short_k_rounds(group, tile):
     assert schedule(group)[:2] == (0, tile)
 
 
+@pytest.mark.parametrize("name,group", [
+    ("chain", [(1 + 7 * i % 65, 1 + 31 * i % 65, 600 + i) for i in range(40)]),
+    ("short", [(1 + 7 * i % 65, 1 + 31 * i % 65, i) for i in range(40)]),
+    ("thin16", [(1 + i % 16, 100 + 29 * i % 160, i % 50) for i in range(500)]),
+    ("thin32", [(1 + i % 32, 100 + 29 * i % 160, i % 50) for i in range(500)]),
+    ("64", [(1 + 53 * i % 300, 1 + 31 * i % 300, i % 50) for i in range(500)]),
+    ("128", [(1280, 1280 - i % 2, 900) for i in range(10)]),
+    ("equal", [(70, 40, 5)] * 900), ("empty", [(0, 4, 4), (4, 0, 4)])])
+def test_tile_table(name, group):
+    """The table: problems with outputs, longest k first, each with its tiles of the chosen shape."""
+    rc, tile, tiles, img = schedule(group)
+    assert rc == 0
+    if name in ("chain", "short", "thin16", "thin32", "64", "128"):
+        assert tile == {"chain": CHAIN, "short": SHORT, "thin16": T16, "thin32": T32, "64": T64, "128": T128}[name]
+    order = sorted((g for g in range(len(group)) if group[g][0] and group[g][1]), key=lambda g: (-max(group[g][2], 1), g))
+    bm, bn = TILE[tile]
+    count = [ceil(group[g][0], bm) * ceil(group[g][1], bn) for g in order]
+    assert tiles == sum(count) == img[0] and img[1] == len(order)
+    assert img[2] == (count[0] if len(set(count)) == 1 else 0)
+    assert img[HDR:HDR + len(order) + 1].tolist() == np.concatenate([[0], np.cumsum(count)]).astype(int).tolist()
+    assert (img[HDR + len(order) + 1:] >> 2).tolist() == order
+
+
 def test_ceil_div(tmp_path):
     """The division that the kernels take their stages, tiles and blocks from."""
     src = tmp_path / "t.cpp"
