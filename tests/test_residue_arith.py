@@ -2,10 +2,9 @@
 on the CPU against exact integer arithmetic (no GPU).
 
 The kernel forms sym(x mod p) of an integer-valued double x with |x| <= T_N from 32-bit digit words
-(exact floor splits), byte dot products against per-modulus weights and one float32 fma that
-floors (u + h) / p.  These tests emulate each step bit for bit:
-  * the float floor is checked exhaustively over every u the dot products can produce and every
-    modulus (a float32 fma is a float64 sum of exact terms, rounded once to float32 here);
+(exact floor splits), byte dot products against per-modulus weights and one float32 fma that rounds
+u / p to an integer in the low bits of the sum with 1.5 2^23 (test_residue_rint.py checks that step
+over every u and modulus).  These tests emulate each step bit for bit:
   * the whole chain is checked against Python integers on edge values (0, +-1, word boundaries,
     powers of two, +-T_N) and random integers of every size up to T_20, for both word layouts;
   * the two-word layout's precondition T_N < 1.5 2^62 holds exactly for N <= 16.
@@ -17,13 +16,7 @@ import numpy as np
 import pytest
 
 MODULI = [256, 255, 253, 251, 247, 239, 233, 229, 227, 223, 217, 211, 199, 197, 193, 191, 181, 179, 173, 167]
-SHIFT = 2048   # the float constant's integer offset; 2048 p = 0 (mod 256)
-
-
-def _consts(p):
-    ipf = np.float32(1.0 / p)
-    cf = np.float32((p // 2 + 0.5) / p + SHIFT)
-    return ipf, cf
+MAGIC = 1.5 * 2.0 ** 23
 
 
 def _sym(r, p):
@@ -37,25 +30,11 @@ def _T(N):
     return math.sqrt(P * 0.5 * (1.0 - 2.0 ** -20)) * (1.0 - 2.0 ** -40)
 
 
-def _floor_q(u, p):
-    """trunc(fmaf(u, ipf, cf)) on int64 arrays u: exact float64 sum, one rounding to float32."""
-    ipf, cf = _consts(p)
-    v = (u.astype(np.float64) * np.float64(ipf) + np.float64(cf)).astype(np.float32)
-    return np.trunc(v).astype(np.int64)
-
-
-@pytest.mark.parametrize("p", MODULI)
-def test_float_floor_exhaustive(p):
-    # unsigned words give [0, 8 * 255^2], the signed word [-4 * 128 * 127, 4 * 128^2]: every u of
-    # both layouts lies in [-2^16, 2^19 + 2^16)
-    u = np.arange(-(1 << 16), (1 << 19) + (1 << 16), dtype=np.int64)
-    q = _floor_q(u, p)
-    h = p // 2
-    assert np.array_equal(q - SHIFT, np.floor_divide(u + h, p))
-    r = u - q * p
-    # r = sym(u mod p) - 2048 p, whose low byte is sym(u mod p)'s
-    assert np.array_equal((r & 0xFF), ((np.floor_divide(u + h, p) * -p + u) & 0xFF))
-    assert np.all((r + SHIFT * p >= -h) & (r + SHIFT * p <= p - 1 - h))
+def _quotient(u, p):
+    """The multiply's 24-bit operand, 2^22 + rint(u / p): the low bits of fmaf(u, 1 / p, 1.5 2^23) for int64
+    arrays u.  float64 holds the sum to 2^-29, far from the half-integers that float32 rounds at."""
+    v = (u * np.float64(np.float32(1.0 / p)) + MAGIC).astype(np.float32)
+    return v.view(np.int32).astype(np.int64) & 0xFFFFFF
 
 
 def _weights(p, q=1):
@@ -91,8 +70,7 @@ def _residue_byte(x, p, q, wide):
     else:
         u += sum(sb(w[1], i) * _sym(e[4 + i], p) for i in range(4))
     assert -(1 << 16) <= u < (1 << 19) + (1 << 16)
-    qq = int(_floor_q(np.array([u]), p)[0])
-    return (u - qq * p) & 0xFF
+    return (u - int(_quotient(np.array([u]), p)[0]) * p) & 0xFF
 
 
 def _edge_values(T):

@@ -4,20 +4,16 @@ u - (2^22 + q) p is that of sym(u mod p)."""
 import numpy as np
 import pytest
 
-from test_residue_arith import MODULI
-
-MAGIC = 1.5 * 2.0 ** 23
+from test_residue_arith import MODULI, _quotient
 
 
 @pytest.mark.parametrize("p", MODULI)
 def test_rint_quotient_exhaustive(p):
     u = np.arange(-(1 << 16), (1 << 19) + (1 << 16), dtype=np.int64)
     ipf = np.float64(np.float32(1.0 / p))
-    # float64 holds u ipf + 1.5 2^23 to 2^-29, far from the half-integers float32 rounds at
-    v = (u * ipf + MAGIC).astype(np.float32)
     if p % 2:
         assert np.abs(np.abs(u * ipf - np.floor(u * ipf)) - 0.5).min() > 2.0 ** -10
-    low = v.view(np.int32).astype(np.int64) & 0xFFFFFF        # the multiply's 24-bit operand
+    low = _quotient(u, p)
     r = u - low * p
     s = u % p
     s = np.where(s > p - 1 - p // 2, s - p, s)
