@@ -13,8 +13,9 @@ Inputs
   --workload G,m,n,k,N[,beta]   a uniform group, for the algorithmic bytes / operations per launch
 
 Calls.  The library's kernels are classified by name into stages (prep, i8_gemm, reconstruct,
-native, memops).  A call starts at every prep kernel, and at a native FP64 kernel that follows
-another native kernel; any other kernel between library kernels ends the current call.  Per call:
+native, memops).  A call starts at every prep kernel (the first, where prep takes two), and at a
+native FP64 kernel that follows another native kernel; any other kernel between library kernels
+ends the current call.  Per call:
   span   first kernel start -> last kernel end
   busy   union of the call's kernel intervals
   gap    span - busy (device idle between the call's kernels)
@@ -49,6 +50,7 @@ _STAGE_RE = [
     (re.compile(r"\bf64_\w*kernel\b"), "native"),
     (re.compile(r"copyBuffer|fillBuffer|__amd_rocclr"), "memops"),
 ]
+_PREP2_RE = re.compile(r"\bresidue_kernel\b")   # prep's second launch, behind norm_kernel
 
 
 # The kernel of each stage that the stage's algorithmic amount is credited to.  The reconstruct
@@ -111,7 +113,8 @@ def split_calls(kernels):
                 calls.append(cur)
                 cur, prev_stage = None, None
             continue
-        new = st == "prep" or (st == "native" and prev_stage == "native") or cur is None
+        second = prev_stage == "prep" and _PREP2_RE.search(name)
+        new = (st == "prep" and not second) or (st == "native" and prev_stage == "native") or cur is None
         if new and cur is not None:
             calls.append(cur)
         if new:

@@ -166,3 +166,14 @@ def test_dot_pass_counts_in_reconstruct_without_roofline(tmp_path):
     recon = 2 * ((3 + 4.0) * 64 * 32 + 8.0 * 64 * 32 + 16.0 * (64 + 32))
     assert by["recon_kernel<true>"]["achieved"] == pytest.approx(recon / 40e-6 / 1e12)
     assert by["dots_kernel"]["stage"] == "reconstruct" and by["dots_kernel"]["achieved"] is None
+
+
+def test_two_launch_prep_is_one_call():
+    """Prep of few rows and columns over a long k takes two kernels; a call starts at the first only."""
+    T = _tool()
+    norm, residue = PREP.replace("prep_kernel", "norm_kernel"), PREP.replace("ggemm::", "void ggemm::", 1).replace("prep_kernel", "residue_kernel<true>")
+    calls = T.split_calls([(norm, 0, 10_000), (residue, 12_000, 40_000), (I8, 40_000, 60_000), (RECON, 60_000, 65_000),
+                           (norm, 70_000, 80_000), (residue, 80_000, 105_000), (I8, 105_000, 125_000), (PREP, 130_000, 140_000)])
+    assert [len(c) for c in calls] == [4, 3, 1]
+    m = T.call_metrics(calls[0])
+    assert (m["span_us"], m["gap_us"], m["prep_us"]) == (65.0, 2.0, 38.0)
