@@ -283,9 +283,10 @@ __global__ void __launch_bounds__(kThreads, OCC) f64_grouped_kernel(const F64Pro
 
 // Few outputs (32 x 32 tiles, 512 threads): waves 0-3 run one
 // accumulator chain each -- 16 x 16 outputs, the whole k -- and waves 4-7, one beside each on its SIMD,
-// stream the operands in stages of BK k, two stages ahead in registers.  A chain takes an MFMA every
-// 64-odd cycles whatever else happens, so the time is k / 4 of them as long as the compute waves issue
-// nothing but fragment reads and MFMAs.
+// stream the operands in stages of BK k, two stages ahead in registers.  The time is that of the chain's
+// k / 4 dependent MFMAs: 64 cycles of the matrix core each, 103 as measured (500x500x60000, 0.73 ms) -- the
+// loader wave's address arithmetic and LDS stores issue on the same SIMD, and a stage's first fragments are
+// read after its barrier.  Compute waves that load for themselves take 145 (64x64x90000 1.42 against 1.01 ms).
 constexpr int kChainTile = 32;
 template <int BK>
 __global__ void __launch_bounds__(2 * kThreads, 2) f64_chain_kernel(const F64Problem* __restrict__ probs,
@@ -414,13 +415,14 @@ int f64_build_schedule(const F64Problem* h, int num, void* h_ws, size_t ws_bytes
   });
 
   // Tile shape.  Microseconds per 16 k, measured on groups of 1 to 3000 tiles: a round of 32 x 32 tiles
-  // (one per compute unit) 0.22, of 64 x 64 tiles 0.58 but at least 0.85 in all, of the thin ones 1.0 but
-  // at least 1.2 (their problems differ in k, and then a round of 32 x 32 ones takes 0.4).  128 x 128
-  // (67 TFLOP/s on long k against 61 of the 64 x 64 tiles) when little of the tiles hangs over the
-  // problems' edges and their rounds of two workgroups per compute unit are nearly filled: a short last
-  // round leaves compute units idle for as long as a full one, unless it has at most one tile for each.
-  // At most one tile per compute unit in all stays on 64 x 64 tiles, four workgroups of which hide each
-  // other's waits: 2048^2 x 2048 323 against 297 us, x 64 23.9 / 21.4, 16 x 512^3 91 / 84.
+  // (one per compute unit) 0.22 with 128-deep stages, 0.20 with 64-deep ones, of 64 x 64 tiles 0.58 but at
+  // least 0.85 in all, of the thin ones 1.0 but at least 1.2 (their problems differ in k, and then a round
+  // of 32 x 32 ones takes 0.4).  128 x 128 (67 TFLOP/s on long k against 61 of the 64 x 64 tiles) when little
+  // of the tiles hangs over the problems' edges and their rounds of two workgroups per compute unit are
+  // nearly filled: a short last round leaves compute units idle for as long as a full one, unless it has
+  // at most one tile for each.  At most one tile per compute unit in all stays on 64 x 64 tiles, four
+  // workgroups of which hide each other's waits: 2048^2 x 2048 323 against 297 us, x 64 23.9 / 21.4,
+  // 16 x 512^3 91 / 84.
   int shape = tile_mode == 128 ? kF64Tile128 : kF64Tile64;
   if (tile_mode == 0 && kmax > 0) {
     auto rounds = [&](int s) { return std::ceil((double)tiles[s] / kCus); };

@@ -749,7 +749,8 @@ __device__ void prep_cols(const oz2_problem& pr, const CrtTables* __restrict__ t
 // of workgroups may share once the shifts are known, the sums of ||dA|| and ||A'|| (walk_*).  Same
 // chains, same order and so the same bits as prep_rows / prep_cols.  Bound by the requests a compute
 // unit keeps in flight: 16 rows x 4 chains per wave, so that each is a whole 128-byte line of A
-// (8 rows x 8 chains, 64 bytes: 267 against 264 us for 2 x 984 rows and columns of 40000), and kDeep to 2 kDeep loads in flight per lane.
+// (8 rows x 8 chains, 64 bytes: 267 against 264 us for 2 x 984 rows and columns of 40000), and kDeep to
+// 2 kDeep loads in flight per lane.
 // f(value, k) over this lane's k = k0, k0 + step, ..., < K of p[k * stride]
 template <int kDeep, class F>
 __device__ __forceinline__ void walk_chain(const GLOBAL double* p, size_t stride, int k0, int step, int K, F f) {
@@ -860,7 +861,7 @@ __device__ void norm_group(const NormOut& o, bool valid, int K, double T, NormSh
   if (o.finite) o.finite[o.i] = nf ? 0 : 1;
 }
 
-// ||dA|| and ||A'|| of 8 rows / 2 columns, from the shifts norm_kernel wrote.
+// ||dA|| and ||A'|| of a workgroup's 32 rows / 8 columns, from the shifts norm_kernel wrote.
 __device__ __forceinline__ void walk_step(double a, int sh, double sc, double& da2, double& na2) {
   const double x = sh >= -1000 && sh <= 1000 ? a * sc : mul_pow2(a, sh), xt = trunc(x), fr = x - xt;
   da2 = fma(fr, fr, da2);
@@ -1054,7 +1055,11 @@ int g_force_split = 0;
 
 // Whether a grouped call's prep takes two launches (norm_kernel, residue_kernel): at most two of the
 // single kernel's workgroups per compute unit without its k splits, each of which reads its rows'
-// whole k again, and enough elements (16 M, 128 MB) that the second launch does not matter.
+// whole k again, and enough elements (16 M, 128 MB) that the second launch does not matter.  us per call
+// in one / two launches (same GPU): 256x256x65536 (40 blocks, 32 M) 1889 / 1286, 2048x1024x8192 (192, 24 M)
+// 717 / 594, 4096x3072x4096 (512, 28 M) 1103 / 1077, 40 x 100x60x5000 (480, 31 M) 602 / 517; past two blocks
+// per compute unit 4096x4096x4096 (640, 32 M) 1373 / 1372, 4096x4096x1024 (640, 8 M) 495 / 511; below 16 M
+// it depends on the blocks: 4096x2048x1024 (384, 6 M) 271 / 278, but 1000x500x4096 (95, 6 M) 211 / 139.
 bool prep_two_pass(long long blocks, long long elems, int cus) { return blocks <= 2LL * cus && elems >= 1LL << 24; }
 
 }  // namespace
