@@ -39,3 +39,30 @@ def test_dense_crossings(rows, cols, beta):
         outs.append([case.C(g).copy() for g in range(2)])
     for a, b in zip(*outs):
         assert same_bits(a, b)
+
+
+@pytest.mark.parametrize("bad", ["rows", "all", "half"])
+@pytest.mark.parametrize("shape", [(88, 80, 300), (80, 121, 257), (64, 17, 129), (17, 16, 300), (336 - 256, 57, 64)])
+def test_dense_edge_tiles(shape, bad):
+    """Tiles over the problem's edge whose entries all (or half of them) take their chains -- rows and
+    columns with an infinity, no summaries: bitwise against the oracle with equal counters, and equal to
+    the handle that defers nothing."""
+    say(f"dense edge tiles {shape}, {bad}")
+    outs = []
+    for form in ("", "tile", "blocks"):
+        case = Case([shape], 23, phi=1.0, beta=0.5)
+        h = case.hp[0]
+        for i in range(0, h.m, 2 if bad == "half" else 1):
+            h.A[i + (3 * i % h.k) * h.lda] = np.inf if i % 3 else -np.inf
+        if bad == "all":
+            for j in range(h.n):
+                h.B[(5 * j) % h.k + j * h.ldb] = np.inf if j % 2 else np.nan
+        case.alloc()
+        env = {"GGEMM_DOT_FORM": form} if form else {}
+        with kernel_handle(case, None, GGEMM_STATS_REPAIR="1", GGEMM_SAFETY_CHAINS="1", **env) as hd:
+            rc, st = run(case, G.PATH_EMU_GROUPED, CFG, handle=hd)
+        assert rc == 0
+        check_case(case, G.PATH_EMU_GROUPED, CFG, st, O.REPAIR_ON)
+        assert st.num_safety_fallback >= h.m * h.n // 2
+        outs.append(case.C(0).copy())
+    assert same_bits(outs[0], outs[1]) and same_bits(outs[0], outs[2])
