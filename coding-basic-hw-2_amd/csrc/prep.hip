@@ -389,7 +389,7 @@ __device__ void prep_rows(const oz2_problem& pr, const CrtTables* __restrict__ t
   // residue role: row rr and W consecutive k, the lanes of a 64-byte k-block of a row side by side, so
   // that a wave's store of a plane covers whole 64-byte lines (1 KB in a row when the planes are
   // packed; with lane = row, half-written lines 64 bytes apart: 64 x 1024^3 per call 2571 -> 2540 us,
-  // 2 x 8192^2 x 16384 33.1 -> 32.6 ms, the residues of 2 x 984 x 40000 with 18 moduli 911 -> 745 us).
+  // the residues of 2 x 984 x 40000 with 18 moduli 911 -> 745 us).
   // Two-word digits: 16 k in one pass; three-word ones: 8 k of both halves of the tile.
   constexpr int W = kWide ? 8 : 16;
   const int rr = kWide ? tid >> 3 : (tid >> 2) & 31;
