@@ -522,9 +522,9 @@ __global__ void __launch_bounds__(kThreads) recon_kernel(const oz2_problem* __re
 // one problem per workgroup: a tile without flags returns after reading its 512 flag bytes;
 // otherwise every flagged entry's dot product is one sequential fma chain over k in ascending order
 // from 0, as the reference's fp64_dot, whichever of three forms computes it:
-//   * dense: when at least a quarter of the tile's entries are flagged (of the ones inside the problem, for
-//     tiles over its edge with more than the compact form takes), the workgroup computes all 4096
-//     chains of the tile at once, each thread a 4 x 4 register block (16 chains), the k-chunks of
+//   * dense: when at least a quarter of the tile's entries are flagged (for a tile over the problem's edge
+//     with more of them than the compact form takes, in two block rows or more: of its entries inside the
+//     problem), the workgroup computes all 4096 chains of the tile at once, each thread a 4 x 4 register block (16 chains), the k-chunks of
 //     A (64 rows) and B (64 columns) double-buffered in LDS and read as 32-byte row / column
 //     quads that a wave's lanes share (broadcast reads): 4 LDS reads per 16 fmas;
 //   * compact: when the flagged entries lie in nR rows and nC columns with nR nC <= kCompactMax,
@@ -1082,11 +1082,14 @@ __global__ void __launch_bounds__(kThreads, 7) dots_kernel(const oz2_problem* __
   // workgroup-uniform: moved to scalar registers, and everything derived from them with them
   const unsigned long long rmask = uniform_u64(rcm[0]), cmask = uniform_u64(rcm[1]);
   const int nR = __popcll(rmask), nC = __popcll(cmask);
-  // A tile over the problem's edge takes the dense form from a quarter of its own entries on, as whole tiles
-  // do: where every entry is flagged (no summaries, or more infinities than they list) deferring the
-  // edge alone put a gather and a crossings GEMM behind the dense tiles' pass -- of the whole matrix when
-  // both edges deferred (336x121x16129, 0.3 % Inf: 3.9 against 2.3 ms per call)
-  dense = dense || (autof && nR * nC > kCompactMax && 4 * total >= min(kRT, m - r0) * min(kRT, pr.n - c0));
+  // A tile over the problem's edge with a quarter of its own entries flagged does not defer: where every
+  // entry is (no summaries, or more infinities than they list), deferring the edge alone put a gather and a
+  // crossings GEMM behind the dense tiles' pass -- of the whole matrix when both edges deferred
+  // (336x121x16129, 0.3 % Inf: 3.9 against 2.3 ms per call).  A wave takes its block column's blocks in
+  // turn, so from two block rows on the dense form is the faster (26x37x4000 all flagged, per call: blocks
+  // 693, dense 517 us), else the blocks (11x63x4000 379, 517).
+  const bool edge = autof && nR * nC > kCompactMax && 4 * total >= min(kRT, m - r0) * min(kRT, pr.n - c0);
+  dense = dense || (edge && rmask >> (__builtin_ctzll(rmask) & ~15) > 0xffffull);   // (edge: rmask != 0)
   if (dense) {
     publish(false);
     dense_dots(pr, r0, c0, fl, buf);
@@ -1097,7 +1100,7 @@ __global__ void __launch_bounds__(kThreads, 7) dots_kernel(const oz2_problem* __
   // however many they are: a tile past the compact form's limit would run them block by block, and
   // one such tile (17 x 16 finite rows and columns of 2048^3 with 0.1 % NaN / Inf) held the whole pass
   // for 0.97 ms of 1.36 (16 x 2048^3 + 2 x 2048^2 x 65536).
-  const bool defer = form == kDotFormAuto && yds[pi].AT && total >= kBandMin && 2 * total >= nR * nC;   // workgroup-uniform
+  const bool defer = form == kDotFormAuto && !edge && yds[pi].AT && total >= kBandMin && 2 * total >= nR * nC;   // workgroup-uniform
   if (defer) {
     publish(true);
     if (t == 0) {

@@ -42,7 +42,7 @@ def test_dense_crossings(rows, cols, beta):
 
 
 @pytest.mark.parametrize("bad", ["rows", "all", "half"])
-@pytest.mark.parametrize("shape", [(88, 80, 300), (80, 121, 257), (64, 17, 129), (17, 16, 300), (336 - 256, 57, 64)])
+@pytest.mark.parametrize("shape", [(88, 80, 300), (80, 121, 257), (64, 17, 129), (17, 16, 300), (16, 57, 300), (11, 24, 129), (80, 57, 64)])
 def test_dense_edge_tiles(shape, bad):
     """Tiles over the problem's edge whose entries all (or half of them) take their chains -- rows and
     columns with an infinity, no summaries: bitwise against the oracle with equal counters, and equal to
