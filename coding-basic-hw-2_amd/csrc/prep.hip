@@ -347,8 +347,10 @@ __device__ void prep_rows(const oz2_problem& pr, const CrtTables* __restrict__ t
     }
     __syncthreads();
     const double rowmax = sm.rowmax[r];
-    // (an infinite row max already makes the shift non-finite: no rescaled second read of the row)
-    const bool resc = valid && isfinite(rowmax) && needs_rescale(rowmax);
+    // (an infinite row max or a NaN already makes the shift non-finite: no rescaled second read of the row;
+    // a row read up to its NaN may not have met its infinities: 2 x 40x40x20000, entries beyond 2^400 and
+    // 0.3 % NaN / Inf, 775 -> 158 us per call)
+    const bool resc = valid && isfinite(rowmax) && needs_rescale(rowmax) && !(trk && sm.nfnan[r]);
     if (resc) {   // rare: exact power-of-two prescaling so the squares cannot overflow / underflow
       const int e = -ilogb(rowmax);
       ss = 0.0;
@@ -604,6 +606,7 @@ __device__ void prep_cols(const oz2_problem& pr, const CrtTables* __restrict__ t
       for (; k < K; k += 32) step(b[k], k);
   }
   if (trk && isnan(ss)) sm.nfnan[w] = 1;   // a sum of squares turns NaN only through a NaN
+  bool nan_col = false;
 #pragma unroll
   for (int o = 16; o; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 32));
   if (trk) {   // every lane's counter update precedes the reads; mx is the largest finite magnitude
@@ -612,9 +615,10 @@ __device__ void prep_cols(const oz2_problem& pr, const CrtTables* __restrict__ t
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     if (lane == 0) sm.nfmx[w] = (unsigned long long)__double_as_longlong(mx);
     if (sm.nfcnt[w] > 0) mx = __builtin_inf();
+    nan_col = sm.nfnan[w] != 0;
   }
-  // (an infinite column max already makes the shift non-finite: no rescaled second read)
-  const bool resc = isfinite(mx) && needs_rescale(mx);
+  // (an infinite column max or a NaN already makes the shift non-finite: no rescaled second read)
+  const bool resc = isfinite(mx) && needs_rescale(mx) && !nan_col;
   if (resc) {
     const int e = -ilogb(mx);
     ss = 0.0;

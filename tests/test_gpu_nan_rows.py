@@ -37,3 +37,30 @@ def test_nan_rows(k, repair, mode):
         rc, st = run(case, G.PATH_EMU_GROUPED, cfg, handle=hd)
     assert rc == 0
     check_case(case, G.PATH_EMU_GROUPED, cfg, st, mode)
+
+
+@pytest.mark.parametrize("k", [255, 1500, 4200])
+@pytest.mark.parametrize("scale_a,scale_b", [(1e280, 1e-300), (1e-290, 1e250)])
+def test_nan_rows_of_extreme_magnitude(k, scale_a, scale_b):
+    """Magnitudes whose squares need the rescaled second read of a row, in rows and columns that hold a
+    NaN, infinities, both in either order, or neither."""
+    say(f"NaN rows of extreme magnitude, k {k}")
+    case = Case([(45, 21, k), (33, 9, k)], 18, phi=1.0, beta=0.5)
+    for h in case.hp:
+        h.A *= scale_a
+        h.B *= scale_b
+        a, b, K = h.lda, h.ldb, h.k
+        h.A[0 + 3 * a], h.A[0 + (K - 2) * a] = np.nan, np.inf
+        h.A[1 + 3 * a], h.A[1 + (K - 2) * a] = -np.inf, np.nan
+        h.A[2 + (K // 2) * a] = np.nan
+        h.A[4 + (K // 2) * a] = np.inf
+        h.B[0], h.B[K - 1] = np.nan, np.inf
+        h.B[b], h.B[b + K - 1] = np.inf, np.nan
+        h.B[2 * b + K // 2] = np.nan
+        h.B[5 * b + K // 2] = -np.inf
+    case.alloc()
+    cfg = G.Config(0, 1e-15, 1, G.REPAIR_ON)
+    with kernel_handle(case, None, GGEMM_STATS_REPAIR="1") as hd:
+        rc, st = run(case, G.PATH_EMU_GROUPED, cfg, handle=hd)
+    assert rc == 0
+    check_case(case, G.PATH_EMU_GROUPED, cfg, st, O.REPAIR_ON)
