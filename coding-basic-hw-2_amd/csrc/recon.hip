@@ -540,6 +540,7 @@ __global__ void __launch_bounds__(kThreads) recon_kernel(const oz2_problem* __re
 // call has them (nf_dot below); only those it cannot decide, and the repairs, take the chains.
 constexpr int kRT = 64;            // tile rows and columns
 constexpr int kDenseMin = 1024;    // flagged entries of a tile from which it takes the dense form
+constexpr int kDenseBlocks = 8;    // blocks with a flag in kWaveDots lanes from which it takes the dense form
 constexpr int kDK = 8;             // dense k-chunk
 constexpr int kSG = 16;            // sparse: entries per group
 constexpr int kListCap = 256;      // sparse list capacity (16 blocks x 3 lanes x 4 entries fit)
@@ -853,7 +854,7 @@ __global__ void __launch_bounds__(kThreads, 7) dots_kernel(const oz2_problem* __
   __shared__ __attribute__((aligned(16))) double buf[kUnion];
   __shared__ uint64_t fl[64];       // flag words of the tile's 16 blocks (4 per block, column-major blocks)
   __shared__ uint32_t list[kListCap];
-  __shared__ int cnt[2];            // flagged entries of the tile, listed entries
+  __shared__ int cnt[3];            // flagged entries of the tile, listed entries, blocks for the block form
   __shared__ unsigned long long rcm[2];   // tile rows / columns holding flagged entries
   __shared__ uint8_t rmap[kRT], cmap[kRT];
   int pi, lt;
@@ -1077,11 +1078,16 @@ __global__ void __launch_bounds__(kThreads, 7) dots_kernel(const oz2_problem* __
     const unsigned long long cbits = ((v | (v >> 16) | (v >> 32) | (v >> 48)) & 0xffffull) << (16 * bj);
     if (rb) atomicOr(&rcm[0], rb);
     if (cbits) atomicOr(&rcm[1], cbits);
+    unsigned long long lanes = v | __shfl_xor((unsigned long long)v, 1);   // lanes of the word's block with a flag
+    lanes |= __shfl_xor(lanes, 2);
+    const int nb = __popcll(__ballot(__popcll(lanes) >= kWaveDots)) >> 2;   // blocks that the block form computes
+    if (t == 0) cnt[2] = nb;
   }
   lds_sync();
   // workgroup-uniform: moved to scalar registers, and everything derived from them with them
   const unsigned long long rmask = uniform_u64(rcm[0]), cmask = uniform_u64(rcm[1]);
   const int nR = __popcll(rmask), nC = __popcll(cmask);
+  const int blocks = __builtin_amdgcn_readfirstlane(cnt[2]);
   // A tile over the problem's edge with a quarter of its own entries flagged does not defer: where every
   // entry is (no summaries, or more infinities than they list), deferring the edge alone put a gather and a
   // crossings GEMM behind the dense tiles' pass -- of the whole matrix when both edges deferred
@@ -1090,17 +1096,12 @@ __global__ void __launch_bounds__(kThreads, 7) dots_kernel(const oz2_problem* __
   // 693, dense 517 us), else the blocks (11x63x4000 379, 517).
   const bool edge = autof && nR * nC > kCompactMax && 4 * total >= min(kRT, m - r0) * min(kRT, pr.n - c0);
   dense = dense || (edge && rmask >> (__builtin_ctzll(rmask) & ~15) > 0xffffull);   // (edge: rmask != 0)
-  if (dense) {
-    publish(false);
-    dense_dots(pr, r0, c0, fl, buf);
-    return;
-  }
   // Dense crossings with enough chains go to the crossings pass, which runs the crossings of all deferred
   // rows and columns of the problem as one GEMM on the matrix cores (needs the gather workspace AT) --
   // however many they are: a tile past the compact form's limit would run them block by block, and
   // one such tile (17 x 16 finite rows and columns of 2048^3 with 0.1 % NaN / Inf) held the whole pass
   // for 0.97 ms of 1.36 (16 x 2048^3 + 2 x 2048^2 x 65536).
-  const bool defer = form == kDotFormAuto && !edge && yds[pi].AT && total >= kBandMin && 2 * total >= nR * nC;   // workgroup-uniform
+  const bool defer = form == kDotFormAuto && !dense && !edge && yds[pi].AT && total >= kBandMin && 2 * total >= nR * nC;   // workgroup-uniform
   if (defer) {
     publish(true);
     if (t == 0) {
@@ -1111,6 +1112,14 @@ __global__ void __launch_bounds__(kThreads, 7) dots_kernel(const oz2_problem* __
     return;
   }
   publish(false);
+  // Half of the tile's blocks and more: the dense form runs at most twice the chains, at once instead of up
+  // to four blocks after another in a wave, and the pass is no longer held by such tiles while others
+  // defer (4000x100x6000 with 2 % of the rows and 10 % of the columns flagged, per call: 3.7 against 2.4 ms).
+  dense = dense || (autof && nR * nC > kCompactMax && blocks >= kDenseBlocks);
+  if (dense) {
+    dense_dots(pr, r0, c0, fl, buf);
+    return;
+  }
   if (autof && nR * nC <= kCompactMax) {   // workgroup-uniform
     if (t < 64) {
       if ((rmask >> t) & 1ull) rmap[__popcll(rmask & ((1ull << t) - 1ull))] = (uint8_t)t;

@@ -66,3 +66,31 @@ def test_dense_edge_tiles(shape, bad):
         assert st.num_safety_fallback >= h.m * h.n // 2
         outs.append(case.C(0).copy())
     assert same_bits(outs[0], outs[1]) and same_bits(outs[0], outs[2])
+
+
+@pytest.mark.parametrize("rows,cols", [(3, 4), (5, 0), (0, 6), (12, 9), (1, 1), (7, 40)])
+def test_flagged_lines(rows, cols):
+    """Whole rows and columns of every 64 x 64 tile take their chains (infinities, no summaries), with some
+    tiles free of either: deferred lines, mixed tiles in the dense form, edge tiles; bitwise against the
+    oracle with equal counters, and equal to the handles that defer nothing / run block by block."""
+    say(f"flagged lines: {rows} rows, {cols} columns per tile")
+    outs = []
+    for form in ("", "tile", "blocks"):
+        case = Case([(150, 200, 300), (64, 128, 65)], 29, phi=1.0, beta=0.5)
+        rng = np.random.default_rng(5)
+        for h in case.hp:
+            for r0 in range(0, h.m, 64):
+                for i in rng.permutation(np.arange(r0, min(r0 + 64, h.m)))[:0 if r0 == 64 else rows]:
+                    h.A[i + (7 * i % h.k) * h.lda] = np.inf
+            for c0 in range(0, h.n, 64):
+                for j in rng.permutation(np.arange(c0, min(c0 + 64, h.n)))[:0 if c0 == 64 else cols]:
+                    h.B[5 * j % h.k + j * h.ldb] = -np.inf if j % 2 else np.nan
+        case.alloc()
+        env = {"GGEMM_DOT_FORM": form} if form else {}
+        with kernel_handle(case, None, GGEMM_STATS_REPAIR="1", GGEMM_SAFETY_CHAINS="1", **env) as hd:
+            rc, st = run(case, G.PATH_EMU_GROUPED, CFG, handle=hd)
+        assert rc == 0
+        check_case(case, G.PATH_EMU_GROUPED, CFG, st, O.REPAIR_ON)
+        outs.append([case.C(g).copy() for g in range(2)])
+    for a, b, c in zip(*outs):
+        assert same_bits(a, b) and same_bits(a, c)
