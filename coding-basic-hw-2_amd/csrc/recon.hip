@@ -521,10 +521,11 @@ __global__ void __launch_bounds__(kThreads) recon_kernel(const oz2_problem* __re
 // uncertified entries) and flags them, one bit per entry.  dots_kernel then covers a 64 x 64 tile of
 // one problem per workgroup: a tile without flags returns after reading its 512 flag bytes;
 // otherwise every flagged entry's dot product is one sequential fma chain over k in ascending order
-// from 0, as the reference's fp64_dot, whichever of three forms computes it:
+// from 0, as the reference's fp64_dot, whichever of these forms computes it:
 //   * dense: when at least a quarter of the tile's entries are flagged (for a tile over the problem's edge
 //     with more of them than the compact form takes, in two block rows or more: of its entries inside the
-//     problem), the workgroup computes all 4096 chains of the tile at once, each thread a 4 x 4 register block (16 chains), the k-chunks of
+//     problem), or half of its 16 x 16 blocks would take the block form, the workgroup computes all 4096
+//     chains of the tile at once, each thread a 4 x 4 register block (16 chains), the k-chunks of
 //     A (64 rows) and B (64 columns) double-buffered in LDS and read as 32-byte row / column
 //     quads that a wave's lanes share (broadcast reads): 4 LDS reads per 16 fmas;
 //   * compact: when the flagged entries lie in nR rows and nC columns with nR nC <= kCompactMax,
@@ -1068,7 +1069,8 @@ __global__ void __launch_bounds__(kThreads, 7) dots_kernel(const oz2_problem* __
   }
   const bool autof = form == kDotFormAuto || form == kDotFormTile;
   bool dense = form == kDotFormDense || (autof && total >= kDenseMin);   // workgroup-uniform
-  if (autof && !dense && t < 64) {   // rows and columns of the flagged entries: word t covers rows 16 bi + 4 q + e, columns 16 bj + c
+  // rows and columns of the flagged entries: word t covers rows 16 bi + 4 q + e, columns 16 bj + c
+  if (autof && !dense && t < 64) {
     const uint64_t v = fl[t];
     const int bi = (t >> 2) & 3, bj = t >> 4, e = t & 3;
     unsigned long long rb = 0ull;
@@ -1101,7 +1103,8 @@ __global__ void __launch_bounds__(kThreads, 7) dots_kernel(const oz2_problem* __
   // however many they are: a tile past the compact form's limit would run them block by block, and
   // one such tile (17 x 16 finite rows and columns of 2048^3 with 0.1 % NaN / Inf) held the whole pass
   // for 0.97 ms of 1.36 (16 x 2048^3 + 2 x 2048^2 x 65536).
-  const bool defer = form == kDotFormAuto && !dense && !edge && yds[pi].AT && total >= kBandMin && 2 * total >= nR * nC;   // workgroup-uniform
+  const bool defer = form == kDotFormAuto && !dense && !edge && yds[pi].AT && total >= kBandMin &&
+                     2 * total >= nR * nC;   // workgroup-uniform
   if (defer) {
     publish(true);
     if (t == 0) {
