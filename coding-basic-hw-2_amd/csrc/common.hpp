@@ -77,8 +77,8 @@ struct F64Problem {
   double alpha, beta;
 };
 
-// ceil(x / b) for every x >= 0: x + b - 1 would wrap for the largest b - 1 sizes an int holds
-__host__ __device__ constexpr int ceil_div(int x, int b) { return x / b + (x % b != 0); }
+// ceil(x / b) for every x >= 0 (as int, x + b - 1 would wrap for the largest b - 1 sizes)
+__host__ __device__ constexpr int ceil_div(int x, int b) { return (int)(((unsigned)x + (unsigned)b - 1u) / (unsigned)b); }
 
 // Schedule image shared by the tile-based kernels (INT8 GEMM, FP64 GEMM):
 //   int[0] total tiles, int[1] entries, int[2] tiles per entry when all entries have the same
